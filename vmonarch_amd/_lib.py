@@ -1,4 +1,5 @@
-"""ctypes binding of libvmonarch_gfx950.so (the C ABI declared in include/vmonarch_amd.h).
+"""ctypes binding of libvmonarch_gfx950.so (the C ABI declared in include/vmonarch_amd.h), and the loader of the host
+module through which the package itself calls it (host()).
 
 torch is imported before the library is loaded so that the process has one HIP runtime:
 the library asks for libamdhip64.so.7 by soname and the dynamic loader hands it the copy torch
@@ -113,6 +114,24 @@ def lib():
             raise RuntimeError(f"vmonarch_amd: library ABI {v}, bindings expect {ABI_VERSION}")
         _lib = L
         return L
+
+
+_host = None
+
+
+def host():
+    """The host module (csrc/host_ops.cpp): torch tensors in, the library's launches out.  Loaded once, after the
+    library and its ABI check."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _vmo_host
+        except ImportError as e:
+            raise RuntimeError(f"vmonarch_amd: the host module is not built or does not load ({e}); run "
+                               "`python -m vmonarch_amd.build`") from e
+        _host = _vmo_host
+    return _host
 
 
 def check(rc, what):

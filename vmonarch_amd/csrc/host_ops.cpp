@@ -1,0 +1,512 @@
+// Host side of the Python package in native code: fills the C ABI's argument structs from torch tensors, allocates
+// results and workspaces from torch's caching allocator and issues the launch sequences of the flash-entropy and
+// VMonarch attention, forward and backward.
+//
+// Why native: a VMonarch forward is six launches plus the fork and join of the recompute's stream.  Issued from
+// Python through ctypes each launch cost ~20 us of host time (struct fields, views, allocations, stream queries)
+// against 4-20 us of GPU time at small sizes, so small calls ran at the host's pace: back to back on one box, a
+// VMonarch forward of a 4 x 64 grid took 135 us and takes 61, of a 16 x 256 grid (batch 2, 4 heads) 139 and 70, a
+// flash-entropy forward (1, 2, 1024, 64) 30 and 17, its training step at (2, 4, 1000, 64) 224 and 115.
+//
+// Every call only issues work on the current stream (and the given side stream, joined before returning); nothing
+// is kept between calls, and no check is cached.  The C ABI it calls (include/vmonarch_amd.h) validates its
+// arguments before launching.
+#include <Python.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/extension.h>
+
+#include <algorithm>
+#include <array>
+#include <optional>
+#include <string>
+#include <tuple>
+#include <utility>
+#include <vector>
+
+#include "../../include/vmonarch_amd.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using OptT = std::optional<Tensor>;
+
+namespace {
+
+[[noreturn]] void raise(PyObject* type, const std::string& msg) {
+  PyErr_SetString(type, msg.c_str());
+  throw py::error_already_set();
+}
+void require(bool ok, const char* msg) {
+  if (!ok) raise(PyExc_AssertionError, msg);
+}
+
+void whole_frames(int64_t nq, int64_t nk, int64_t frames) {
+  if (frames == 0) raise(PyExc_ZeroDivisionError, "no frames");
+  require(nq % frames == 0 && nk % frames == 0, "whole frames");
+}
+
+int dtype_code(const Tensor& t) {
+  if (t.scalar_type() == at::kBFloat16) return VMO_DTYPE_BF16;
+  if (t.scalar_type() == at::kHalf) return VMO_DTYPE_F16;
+  raise(PyExc_KeyError, std::string("torch.") + c10::toString(t.scalar_type()));
+}
+
+// (B, H, N, F) tensor -> view (element strides, feature dim contiguous)
+vmo_view view(const Tensor& t) {
+  require(t.dim() == 4 && t.stride(3) == 1, "feature dimension must be contiguous");
+  return vmo_view{t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)};
+}
+
+// t itself when its rows are 16-byte aligned with a contiguous feature dim, else a contiguous copy
+Tensor row_aligned(const Tensor& t) {
+  bool ok = t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  for (int64_t d = 0; ok && d < t.dim() - 1; ++d) ok = t.stride(d) % 8 == 0;
+  return ok ? t : t.contiguous();
+}
+
+using Order = std::array<int, 3>;
+// order of t's (B, H, N) dims in memory, outermost first (by stride)
+Order layout_order(const Tensor& t) {
+  Order o{0, 1, 2};
+  std::stable_sort(o.begin(), o.end(), [&](int a, int b) { return t.stride(a) > t.stride(b); });
+  return o;
+}
+// an uninitialised (B, H, N, feat) tensor whose (B, H, N) dims lie in memory in `order`, feature dim innermost
+Tensor empty_in_order(const Order& order, const int64_t (&dims)[3], int64_t feat, const at::TensorOptions& opt) {
+  int64_t st[3], s = feat;
+  for (int i = 2; i >= 0; --i) {
+    st[order[i]] = s;
+    s *= std::max<int64_t>(dims[order[i]], 1);   // (torch's strides of an empty dim)
+  }
+  return at::empty_strided({dims[0], dims[1], dims[2], feat}, {st[0], st[1], st[2], 1}, opt);
+}
+Tensor empty_in_layout(const Tensor& ref, int64_t feat) {
+  const int64_t dims[3] = {ref.size(0), ref.size(1), ref.size(2)};
+  return empty_in_order(layout_order(ref), dims, feat, ref.options());
+}
+at::TensorOptions f32(const Tensor& t) { return t.options().dtype(at::kFloat); }
+
+void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+void check(int rc, const char* what) {
+  if (rc != 0)
+    raise(PyExc_RuntimeError, std::string(what) + " failed (code " + std::to_string(rc) + "): " + vmo_last_error());
+}
+
+// ---- single launches -------------------------------------------------------------------------------------------
+
+// q: F*nq rows; k, w0, w1: F*nk rows; o, lse, ent optional outputs.  rows >= 0: only the first `rows` queries.
+struct FwdCall {
+  const Tensor &q, &k, &w0;
+  const Tensor* w1;
+  double sm_scale;
+  int64_t frames;
+  const Tensor &o;
+  const Tensor* lse;
+  const Tensor* ent;
+  int64_t splits;
+  bool fp8;
+  int64_t rows;
+};
+vmo_fea_fwd_args fwd_args(const FwdCall& c) {
+  vmo_fea_fwd_args a{};
+  a.dtype = dtype_code(c.q);
+  a.batch = c.q.size(0); a.heads = c.q.size(1); a.frames = c.frames;
+  const int64_t nq = c.rows >= 0 ? c.rows : c.q.size(2), nk = c.k.size(2);
+  whole_frames(nq, nk, c.frames);
+  a.nq = nq / c.frames; a.nk = nk / c.frames;
+  a.d = c.q.size(3); a.dw0 = c.w0.size(3); a.dw1 = c.w1 ? c.w1->size(3) : 0;
+  a.q = view(c.q); a.k = view(c.k); a.w0 = view(c.w0); a.o = view(c.o);
+  if (c.w1) a.w1 = view(*c.w1);
+  if (c.lse) a.lse = c.lse->data_ptr<float>();
+  if (c.ent) a.ent = c.ent->data_ptr<float>();
+  if (c.lse && c.ent)
+    require(c.lse->stride(0) == c.ent->stride(0) && c.lse->stride(1) == c.ent->stride(1), "lse and ent strides");
+  if (const Tensor* st = c.lse ? c.lse : c.ent) {
+    require(st->stride(2) == 1, "lse / ent token stride");
+    a.stat_stride_b = st->stride(0); a.stat_stride_h = st->stride(1);
+  }
+  a.sm_scale = (float)c.sm_scale;
+  a.num_splits = (int32_t)c.splits;
+  a.qk_fp8 = c.fp8;
+  return a;
+}
+Tensor workspace(size_t bytes, const Tensor& like) { return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte)); }
+// launched on `stream`; returns the workspace (undefined when none is needed), which must outlive the work: on the
+// current stream the caching allocator sees to that, on another the caller keeps it until it has joined that stream
+Tensor run_fwd(const FwdCall& c, void* stream) {
+  vmo_fea_fwd_args a = fwd_args(c);
+  Tensor ws;
+  if (const size_t bytes = vmo_fea_fwd_workspace_size(&a)) {
+    ws = workspace(bytes, c.q);
+    a.workspace = ws.data_ptr();
+    a.workspace_bytes = bytes;
+  }
+  check(vmo_fea_fwd(&a, stream), "vmo_fea_fwd");
+  return ws;
+}
+const Tensor* ptr(const OptT& t) { return t ? &*t : nullptr; }
+
+std::tuple<Tensor, OptT, OptT> fea_fwd(const Tensor& q, const Tensor& k, const Tensor& w0, const OptT& w1, double sm_scale,
+                                       int64_t frames, OptT o, OptT lse, OptT ent, bool want_ent, bool want_lse,
+                                       int64_t num_splits, bool qk_fp8) {
+  const int64_t B = q.size(0), H = q.size(1), NQ = q.size(2);
+  if (!o) o = at::empty({B, H, NQ, w0.size(3) + (w1 ? w1->size(3) : 0)}, q.options());
+  if (!lse && want_lse) lse = at::empty({B, H, NQ}, f32(q));
+  if (!ent && want_ent) ent = at::empty({B, H, NQ}, f32(q));
+  run_fwd({q, k, w0, ptr(w1), sm_scale, frames, *o, ptr(lse), ptr(ent), num_splits, qk_fp8, -1}, stream_of(q));
+  return {*o, lse, ent};
+}
+
+struct BwdCall {
+  const Tensor &q, &k, &v, &o, &lse, &ent, &dO, &dE;
+  double sm_scale;
+  const Tensor *dq, *dk, *dv, *v1;
+  int64_t frames;
+  int32_t flags;
+  const Tensor *dq_base, *dk_base, *dv_base, *delta;
+  int64_t rows;   // >= 0: only the first `rows` queries
+};
+void run_bwd(const BwdCall& c) {
+  vmo_fea_bwd_args a{};
+  a.flags = c.flags;
+  a.dtype = dtype_code(c.q);
+  const int64_t nq = c.rows >= 0 ? c.rows : c.q.size(2), nk = c.k.size(2);
+  whole_frames(nq, nk, c.frames);
+  a.batch = c.q.size(0); a.heads = c.q.size(1); a.nq = nq / c.frames; a.nk = nk / c.frames;
+  a.d = c.q.size(3); a.dv = c.v.size(3) * (c.v1 ? 2 : 1); a.frames = c.frames;
+  a.q = view(c.q); a.k = view(c.k); a.v = view(c.v); a.o = view(c.o); a.grad_o = view(c.dO);
+  a.grad_q = view(*c.dq); a.grad_k = view(*c.dk);
+  if (c.dv) a.grad_v = view(*c.dv);
+  auto base = [](const Tensor* b, const Tensor* g, vmo_view& out) {
+    if (!b) return;
+    require(g && b->sizes() == g->sizes(), "a base is shaped like its gradient");
+    out = view(*b);
+  };
+  base(c.dq_base, c.dq, a.grad_q_base); base(c.dk_base, c.dk, a.grad_k_base); base(c.dv_base, c.dv, a.grad_v_base);
+  require(c.lse.strides() == c.ent.strides() && c.lse.stride(2) == 1 && c.dE.stride(2) == 1, "lse / ent / de strides");
+  a.lse = c.lse.data_ptr<float>(); a.ent = c.ent.data_ptr<float>(); a.grad_ent = c.dE.data_ptr<float>();
+  a.stat_stride_b = c.lse.stride(0); a.stat_stride_h = c.lse.stride(1);
+  a.grad_ent_stride_b = c.dE.stride(0); a.grad_ent_stride_h = c.dE.stride(1);
+  a.sm_scale = (float)c.sm_scale;
+  if (c.v1) {
+    require(c.v1->sizes() == c.v.sizes() && c.v1->strides() == c.v.strides() && c.v1->dtype() == c.v.dtype(),
+            "v1 has the shape, strides and dtype of v");
+    a.v1 = view(*c.v1); a.dv1 = c.v1->size(3);
+  }
+  if (c.delta) {
+    require(c.delta->scalar_type() == at::kFloat && c.delta->stride(2) == 1, "delta: float32, unit token stride");
+    a.delta = c.delta->data_ptr<float>();
+    a.delta_stride_b = c.delta->stride(0); a.delta_stride_h = c.delta->stride(1);
+  }
+  const size_t bytes = vmo_fea_bwd_workspace_size(&a);
+  const Tensor ws = workspace(bytes, c.q);
+  a.workspace = ws.data_ptr(); a.workspace_bytes = bytes;
+  check(vmo_fea_bwd(&a, stream_of(c.q)), "vmo_fea_bwd");
+}
+
+std::tuple<Tensor, Tensor, OptT> fea_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse,
+                                         const Tensor& ent, const Tensor& dO, const Tensor& dE, double sm_scale, OptT dq,
+                                         OptT dk, OptT dv, const std::string& overwrite, const OptT& v1, bool fold_k,
+                                         const OptT& dk_base, const OptT& dv_base, int64_t frames, int64_t route_flags,
+                                         const OptT& dq_base, const OptT& delta) {
+  int32_t flags = (fold_k ? VMO_BWD_FOLD_K : 0) | (int32_t)route_flags;
+  struct G { const OptT& t; char name; int accum, f32_bit, sum; const OptT& base; };
+  for (const G& g : {G{dq, 'q', VMO_BWD_ACCUM_Q, VMO_BWD_F32_Q, VMO_BWD_SUM_Q, dq_base},
+                     G{dk, 'k', VMO_BWD_ACCUM_K, VMO_BWD_F32_K, VMO_BWD_SUM_K, dk_base},
+                     G{dv, 'v', VMO_BWD_ACCUM_V, VMO_BWD_F32_V, VMO_BWD_SUM_V, dv_base}}) {
+    if (g.base) {
+      require(g.base->scalar_type() == at::kFloat && (!g.t || g.t->scalar_type() == q.scalar_type()),
+              "base fp32, result q.dtype");
+      flags |= g.sum;
+    } else if (g.t && g.t->scalar_type() != q.scalar_type()) {
+      require(g.t->scalar_type() == at::kFloat, "a gradient passed in must be float32 or q's dtype");
+      flags |= overwrite.find(g.name) != std::string::npos ? g.f32_bit : g.accum;
+    }
+  }
+  const int64_t B = q.size(0), H = q.size(1), NQ = q.size(2), NK = k.size(2), D = q.size(3);
+  if (!dq) dq = at::empty({B, H, NQ, D}, q.options());
+  if (!dk) dk = at::empty({B, H, NK, D}, q.options());
+  if (!dv && !(fold_k && !v1))
+    dv = at::empty({B, H, NK, fold_k ? v1->size(3) : v.size(3) * (v1 ? 2 : 1)}, q.options());
+  run_bwd({q, k, v, o, lse, ent, dO, dE, sm_scale, ptr(dq), ptr(dk), ptr(dv), ptr(v1), frames, flags, ptr(dq_base),
+           ptr(dk_base), ptr(dv_base), ptr(delta), -1});
+  return {*dq, *dk, dv};
+}
+
+void lstep_fwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tensor& res, int64_t m, int64_t b, double scale,
+               bool last, int64_t skip, double min_col_mass) {
+  vmo_lstep_args a{};
+  a.dtype = dtype_code(q);
+  a.batch = q.size(0); a.heads = q.size(1); a.num_blocks = m; a.block_size = b;
+  a.d = q.size(3); a.dv = last ? out.size(3) - q.size(3) : 0;
+  a.last = last; a.skip_tokens = (int32_t)skip;
+  a.q = view(q); a.out = view(out); a.res = view(res);
+  a.ent = ent.data_ptr<float>();
+  a.ent_stride_b = ent.stride(0); a.ent_stride_h = ent.stride(1);
+  a.scale = (float)scale; a.min_col_mass = (float)min_col_mass;
+  check(vmo_lstep_fwd(&a, stream_of(q)), "vmo_lstep_fwd");
+}
+
+void lstep_bwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tensor& grad_res, const Tensor& grad_q,
+               const Tensor& grad_out, int64_t m, int64_t b, double scale, bool last, int64_t skip, double min_col_mass,
+               bool overwrite_q, const OptT& delta) {
+  vmo_lstep_bwd_args a{};
+  a.dtype = dtype_code(q);
+  a.batch = q.size(0); a.heads = q.size(1); a.num_blocks = m; a.block_size = b;
+  a.d = q.size(3); a.dv = last ? out.size(3) - q.size(3) : 0;
+  a.last = last; a.skip_tokens = (int32_t)skip;
+  a.q = view(q); a.out = view(out); a.grad_res = view(grad_res); a.grad_q = view(grad_q); a.grad_out = view(grad_out);
+  a.ent = ent.data_ptr<float>();
+  a.ent_stride_b = ent.stride(0); a.ent_stride_h = ent.stride(1);
+  a.scale = (float)scale; a.min_col_mass = (float)min_col_mass;
+  a.flags = overwrite_q ? VMO_LSTEP_BWD_OVERWRITE_Q : 0;
+  if (delta) {
+    require(delta->scalar_type() == at::kFloat && delta->stride(2) == 1, "delta: float32, unit token stride");
+    a.delta = delta->data_ptr<float>();
+    a.delta_stride_b = delta->stride(0); a.delta_stride_h = delta->stride(1);
+  }
+  check(vmo_lstep_bwd(&a, stream_of(q)), "vmo_lstep_bwd");
+}
+
+// ---- flash-entropy attention (all N rows valid, head dims the kernels take as they are) --------------------------
+
+std::tuple<Tensor, Tensor, Tensor> fea_attention(const Tensor& q0, const Tensor& k0, const Tensor& v0, double sm_scale) {
+  const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0);
+  const int64_t B = q.size(0), H = q.size(1), N = q.size(2);
+  Tensor o = empty_in_layout(q0, v.size(3));
+  Tensor lse = at::empty({B, H, N}, f32(q)), ent = at::empty({B, H, N}, f32(q));
+  if (N > 0) run_fwd({q, k, v, nullptr, sm_scale, 1, o, &lse, &ent, 1, false, -1}, stream_of(q));
+  return {o, ent, lse};
+}
+
+std::tuple<Tensor, Tensor, Tensor> fea_attention_bwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor& o0,
+                                                     const Tensor& lse, const Tensor& ent, const Tensor& do0,
+                                                     const Tensor& dE, double sm_scale) {
+  // the gradients in the memory order of the caller's q, k, v
+  Tensor dq = empty_in_layout(q0, q0.size(3)), dk = empty_in_layout(k0, k0.size(3)), dv = empty_in_layout(v0, v0.size(3));
+  const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0), o = row_aligned(o0), dO = row_aligned(do0);
+  run_bwd({q, k, v, o, lse, ent, dO, dE, sm_scale, &dq, &dk, &dv, nullptr, 1, 0, nullptr, nullptr, nullptr, nullptr, -1});
+  return {dq, dk, dv};
+}
+
+// ---- VMonarch attention ------------------------------------------------------------------------------------------
+
+// A side stream's work between fork (it waits for the current stream) and join (the current stream waits for it).
+struct SideStream {
+  hipStream_t main, side;
+  bool open = false;
+  SideStream(void* m, int64_t s) : main((hipStream_t)m), side((hipStream_t)s) {}
+  SideStream(const SideStream&) = delete;
+  ~SideStream() {   // an error between fork and join: joined all the same, before the workspaces are given back
+    if (!open) return;
+    try { join(); } catch (py::error_already_set&) {}
+  }
+  static void order(hipStream_t after, hipStream_t then) {   // work issued to `then` from here on follows `after`'s
+    hipEvent_t e;
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) raise(PyExc_RuntimeError, "vmonarch: no event");
+    hipError_t rc = hipEventRecord(e, after);
+    if (rc == hipSuccess) rc = hipStreamWaitEvent(then, e, 0);
+    (void)hipEventDestroy(e);   // (released once the recorded work is done)
+    if (rc != hipSuccess) raise(PyExc_RuntimeError, std::string("vmonarch: stream order: ") + hipGetErrorString(rc));
+  }
+  void fork() {
+    order(main, side);
+    open = true;
+  }
+  void join() {
+    open = false;
+    order(side, main);
+  }
+};
+
+// Where the recompute runs: on the caller's stream after the chain, or on the side stream, forked at the start,
+// after R-step 0 or after the last R-step.
+enum Overlap { kOff = 0, kStart = 1, kAfterR0 = 2, kAfterR1 = 3 };
+
+struct Stages {   // the caller's stage hook (None: none), with the torch stream objects it is told of
+  py::object hook, main, side;
+  void operator()(const char* name, int it, const char* phase, bool on_side = false) const {
+    if (!hook.is_none()) hook(it < 0 ? std::string(name) : name + std::to_string(it), phase, on_side ? side : main);
+  }
+};
+
+Tensor vmonarch_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, int64_t m, int64_t b, int64_t iters,
+                    int64_t recompute_tokens, double min_col_mass, double scale, bool qk_fp8, int64_t splits, int overlap,
+                    int64_t side_handle, py::object hook, py::object main_obj, py::object side_obj) {
+  const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0);
+  const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Dv = v.size(3);
+  const int64_t rt = std::min<int64_t>(recompute_tokens, N);
+  const Stages stage{std::move(hook), std::move(main_obj), std::move(side_obj)};
+  void* const main = stream_of(q);
+  Tensor ent = at::empty({B, H, N}, f32(q));
+  Tensor z = empty_in_layout(q, Dv);   // in the caller's layout
+  Tensor ws;                           // the recompute's workspace: held until its stream is joined
+  SideStream ss(main, side_handle);
+  // exact attention of the first rt queries, into rows of z that the L-steps do not write
+  auto recompute = [&](void* stream, bool on_side) {
+    stage("recompute", -1, "begin", on_side);
+    ws = run_fwd({q, k, v, nullptr, scale, 1, z, nullptr, nullptr, splits, false, rt}, stream);
+    stage("recompute", -1, "end", on_side);
+  };
+  bool forked = false;
+  auto fork = [&] {
+    forked = true;
+    ss.fork();   // q, k, v and z are ready on the caller's stream
+    recompute((void*)ss.side, true);
+  };
+  if (rt > 0 && overlap == kStart) fork();
+  Tensor u, out;
+  for (int64_t it = 0; it < iters; ++it) {
+    const bool last = it == iters - 1;
+    out = at::empty({B, H, N, D + (last ? Dv : 0)}, q.options());
+    stage("rstep", it, "begin");   // iteration 0 folds u = q * scale into the softmax scale
+    run_fwd({it == 0 ? q : u, k, k, last ? &v : nullptr, it == 0 ? scale : 1.0, m, out, nullptr, &ent, 1, qk_fp8, -1}, main);
+    stage("rstep", it, "end");
+    if (rt > 0 && !forked && ((overlap == kAfterR0 && it == 0) || (overlap == kAfterR1 && last))) fork();
+    stage("lstep", it, "begin");
+    if (last) {
+      lstep_fwd(q, out, ent, z, m, b, scale, true, rt, min_col_mass);
+    } else {
+      if (!u.defined()) u = at::empty({B, H, N, D}, q.options());
+      lstep_fwd(q, out, ent, u, m, b, scale, false, 0, min_col_mass);
+    }
+    stage("lstep", it, "end");
+  }
+  if (rt > 0) {
+    if (forked) ss.join();   // z is complete on the caller's stream
+    else recompute(main, false);
+  }
+  return z;
+}
+
+// The forward that keeps what the backward needs: (orders, q, k, v, z, lse_rt, [x, out, lse, ent] per iteration).
+std::tuple<std::vector<int>, std::vector<Tensor>> vmonarch_fwd_train(const Tensor& q0, const Tensor& k0, const Tensor& v0,
+                                                                     int64_t m, int64_t b, int64_t iters, int64_t rt,
+                                                                     double min_col_mass, double scale, int64_t splits,
+                                                                     bool overlap, int64_t side_handle) {
+  std::vector<int> orders;
+  for (const Tensor* t : {&q0, &k0, &v0})
+    for (int d : layout_order(*t)) orders.push_back(d);
+  Tensor z = empty_in_layout(q0, v0.size(3));
+  // read in place in any memory order: the kernels take each head's m frames as m problems
+  Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0);
+  if (k.strides() != v.strides()) {   // the backward reads the values [k | v] as two parts with one set of strides
+    k = k.contiguous();
+    v = v.contiguous();
+  }
+  const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Dv = v.size(3);
+  void* const main = stream_of(q);
+  Tensor lse_rt, ws;
+  SideStream ss(main, side_handle);
+  if (rt > 0) lse_rt = at::empty({B, H, rt}, f32(q));
+  auto recompute = [&](void* stream) {
+    ws = run_fwd({q, k, v, nullptr, scale, 1, z, &lse_rt, nullptr, splits, false, rt}, stream);
+  };
+  if (rt > 0 && overlap) {
+    ss.fork();
+    recompute((void*)ss.side);
+  }
+  std::vector<Tensor> saved;
+  Tensor u;
+  for (int64_t it = 0; it < iters; ++it) {
+    const bool last = it == iters - 1;
+    Tensor out = at::empty({B, H, N, D + (last ? Dv : 0)}, q.options());
+    Tensor lse = at::empty({B, H, N}, f32(q)), ent = at::empty({B, H, N}, f32(q));
+    const Tensor x = it == 0 ? q : u;
+    run_fwd({x, k, k, last ? &v : nullptr, it == 0 ? scale : 1.0, m, out, &lse, &ent, 1, false, -1}, main);
+    if (last) {
+      lstep_fwd(q, out, ent, z, m, b, scale, true, rt, min_col_mass);
+    } else {
+      u = at::empty({B, H, N, D}, q.options());
+      lstep_fwd(q, out, ent, u, m, b, scale, false, 0, min_col_mass);
+    }
+    for (const Tensor& t : {x, out, lse, ent}) saved.push_back(t);
+  }
+  if (rt > 0) {
+    if (overlap) ss.join();   // z and lse_rt are complete on the caller's stream
+    else recompute(main);
+  }
+  std::vector<Tensor> all{q, k, v, z, rt > 0 ? lse_rt : at::empty({0}, q.options())};
+  all.insert(all.end(), saved.begin(), saved.end());
+  return {orders, all};
+}
+
+// Call order: the L- and R-step backwards from the last iteration down, R-step 0's last of all and the recompute's
+// (rows [0, rt), vmonarch.py:66-68) just before it.  Every gradient is written once, in the caller's dtype and
+// memory order, by the last call that contributes to it: the fp32 sum of the earlier contributions plus its own
+// (VMO_BWD_SUM_*), so no conversion pass follows.  dq: the L-steps (the first overwrites, the rest add), the
+// recompute, then R-step 0 (x = q).  dk: every R-step (values start with k: the kernels fold k's value-role
+// gradient into dk, as autograd's sum over k's uses at vmonarch.py:50 does), the recompute, R-step 0 last.  dv: the
+// last R-step (values [k | v]) and the recompute.
+std::tuple<Tensor, Tensor, Tensor> vmonarch_bwd(const std::vector<int>& orders, const std::vector<Tensor>& all, const Tensor& dz0,
+                                                int64_t m, int64_t b, int64_t iters, int64_t rt, double min_col_mass,
+                                                double scale, bool want_delta) {
+  const Tensor &q = all[0], &k = all[1], &v = all[2], &z = all[3], &lse_rt = all[4];
+  const Tensor dz = row_aligned(dz0.to(q.scalar_type()));
+  const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Dv = v.size(3);
+  const int64_t dims[3] = {B, H, N};
+  auto grad = [&](int i, int64_t feat) {
+    return empty_in_order(Order{orders[3 * i], orders[3 * i + 1], orders[3 * i + 2]}, dims, feat, q.options());
+  };
+  Tensor gq = grad(0, D), gk = grad(1, D), gv = grad(2, Dv);
+  Tensor dq = at::empty({B, H, N, D}, f32(q));
+  struct Sum {   // one gradient's fp32 partial sum and final tensor
+    Tensor partial, result;
+    bool started;
+  } sk{at::empty({B, H, N, D}, f32(q)), gk, false}, sv{at::empty({B, H, N, Dv}, f32(q)), gv, false};
+  const Tensor de = at::zeros({B, H, N}, f32(q));
+  // rowsum(out * d out), formed by the L-step backward that writes d out and read by the R-step backward in place of
+  // another pass over both
+  OptT delta;
+  if (want_delta) delta = at::empty({B, H, N}, f32(q));
+  // where one call puts its part of a gradient: into the fp32 partial sum (the first call overwrites it), or from
+  // its last contribution into the result
+  struct Put { const Tensor* g; const Tensor* base; int32_t flags; };
+  auto put = [](Sum& s, bool last_writer, int accum, int f32_bit, int sum) {
+    if (last_writer) return Put{&s.result, s.started ? &s.partial : nullptr, s.started ? sum : 0};
+    const bool first = !s.started;
+    s.started = true;
+    return Put{&s.partial, nullptr, first ? f32_bit : accum};
+  };
+  auto put_k = [&](bool lw) { return put(sk, lw, VMO_BWD_ACCUM_K, VMO_BWD_F32_K, VMO_BWD_SUM_K); };
+  auto put_v = [&](bool lw) { return put(sv, lw, VMO_BWD_ACCUM_V, VMO_BWD_F32_V, VMO_BWD_SUM_V); };
+  Tensor g = dz;
+  for (int64_t it = iters - 1; it >= 0; --it) {
+    const bool last = it == iters - 1;
+    const Tensor &x = all[5 + 4 * it], &out = all[6 + 4 * it], &lse = all[7 + 4 * it], &ent = all[8 + 4 * it];
+    Tensor dout = at::empty_like(out);
+    lstep_bwd(q, out, ent, g, dq, dout, m, b, scale, last, last ? rt : 0, min_col_mass, last, delta);
+    if (it == 0 && rt > 0) {   // the exact attention of the first rt queries; it reads every key and value
+      const Tensor zeros = de.narrow(2, 0, rt);
+      const Tensor ent0 = lse_rt;   // (multiplied by a zero entropy gradient)
+      const Put pk = put_k(false), pv = put_v(iters > 1);
+      run_bwd({q, k, v, z, lse_rt, ent0, dz, zeros, scale, &dq, pk.g, pv.g, nullptr, 1, VMO_BWD_ACCUM_Q | pk.flags | pv.flags,
+               nullptr, pk.base, pv.base, nullptr, rt});
+    }
+    // values k, or [k | v] read from the two tensors in place (vmonarch.py:50); m frames per head
+    const Put pk = put_k(it == 0);
+    Put pv{nullptr, nullptr, 0};
+    if (last) pv = put_v(iters == 1 || rt == 0);
+    Tensor gx;
+    if (it > 0) gx = at::empty({B, H, N, D}, q.options());
+    run_bwd({x, k, k, out, lse, ent, dout, de, it == 0 ? scale : 1.0, it == 0 ? &gq : &gx, pk.g, pv.g, last ? &v : nullptr, m,
+             VMO_BWD_FOLD_K | pk.flags | pv.flags | (it == 0 ? VMO_BWD_SUM_Q : 0), it == 0 ? &dq : nullptr, pk.base, pv.base,
+             ptr(delta), -1});
+    if (it > 0) g = gx;   // dL/du of the previous L-step's output
+  }
+  return {gq, gk, gv};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
+  mod.def("fea_fwd", &fea_fwd);
+  mod.def("fea_bwd", &fea_bwd);
+  mod.def("lstep_fwd", &lstep_fwd);
+  mod.def("lstep_bwd", &lstep_bwd);
+  mod.def("fea_attention", &fea_attention);
+  mod.def("fea_attention_bwd", &fea_attention_bwd);
+  mod.def("vmonarch_fwd", &vmonarch_fwd);
+  mod.def("vmonarch_fwd_train", &vmonarch_fwd_train);
+  mod.def("vmonarch_bwd", &vmonarch_bwd);
+}

@@ -1,7 +1,7 @@
 """FlashEntropyAttention: attention that also returns the entropy of every attention row.
 
 Drop-in for video_monarch_attention/kernel.py (reference).  Same public function and autograd
-contract; the body calls the gfx950 HIP kernels through the C ABI (vmonarch_amd/_lib.py).
+contract; the body calls the gfx950 HIP kernels through the host module (csrc/host_ops.cpp).
 
 Differences from the reference that callers can observe: none in values (within bf16
 tolerance).  Internally there is no padding to a multiple of 128 (kernel.py:399-400): tails are
@@ -39,44 +39,7 @@ def fea_forward(q, k, w0, w1, sm_scale, frames=1, o=None, lse=None, ent=None, wa
     to write into; lse / ent views need a unit token stride.  `qk_fp8`: S = q k^T in fp8 (the VMonarch
     R-step variants only; vmo_fea_fwd_args.qk_fp8).
     """
-    L = _lib.lib()
-    B, H, NQ, D = q.shape
-    NK = k.shape[2]
-    assert NQ % frames == 0 and NK % frames == 0
-    dw0 = w0.shape[-1]
-    dw1 = 0 if w1 is None else w1.shape[-1]
-    dev = q.device
-    if o is None:
-        o = torch.empty((B, H, NQ, dw0 + dw1), device=dev, dtype=q.dtype)
-    if lse is None and want_lse:
-        lse = torch.empty((B, H, NQ), device=dev, dtype=torch.float32)
-    if ent is None and want_ent:
-        ent = torch.empty((B, H, NQ), device=dev, dtype=torch.float32)
-    st = lse if lse is not None else ent
-    if lse is not None and ent is not None:
-        assert lse.stride()[:2] == ent.stride()[:2]
-    a = _lib.FeaFwdArgs()
-    a.dtype = _lib.DTYPES[q.dtype]
-    a.batch, a.heads, a.frames = B, H, frames
-    a.nq, a.nk = NQ // frames, NK // frames
-    a.d, a.dw0, a.dw1 = D, dw0, dw1
-    a.q, a.k, a.w0, a.o = _lib.view(q), _lib.view(k), _lib.view(w0), _lib.view(o)
-    a.w1 = _lib.view(w1) if w1 is not None else _lib.View(0, 0, 0, 0)
-    a.lse = lse.data_ptr() if lse is not None else None
-    a.ent = ent.data_ptr() if ent is not None else None
-    if st is not None:
-        assert st.stride(2) == 1
-        a.stat_stride_b, a.stat_stride_h = st.stride(0), st.stride(1)
-    a.sm_scale = float(sm_scale)
-    a.num_splits = int(num_splits)
-    a.qk_fp8 = int(bool(qk_fp8))
-    ws = None
-    nbytes = L.vmo_fea_fwd_workspace_size(a)
-    if nbytes:
-        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-        a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
-    _lib.check(L.vmo_fea_fwd(a, _lib.stream_of(q)), "vmo_fea_fwd")
-    return o, lse, ent
+    return _lib.host().fea_fwd(q, k, w0, w1, sm_scale, frames, o, lse, ent, want_ent, want_lse, num_splits, bool(qk_fp8))
 
 
 class _FlashEntropyAttention(torch.autograd.Function):
@@ -99,6 +62,12 @@ class _FlashEntropyAttention(torch.autograd.Function):
             raise RuntimeError("vmonarch_amd: flash_entropy_attention needs GPU tensors (no CPU path)")
         n = int(n_valid)
         Dk, Dvk = _kernel_widths(D, Dv)
+        ctx.sm_scale = sm_scale
+        ctx.n_valid = n
+        if n == N and Dvk == Dv:   # no padding rows, no padded features
+            o, ent, lse = _lib.host().fea_attention(q, k, v, sm_scale)
+            ctx.save_for_backward(q, k, v, o, lse, ent)
+            return o, ent
         qx, kx, vx = (_lib.row_aligned(_pad_features(t[:, :, :n], w)) for t, w in ((q, Dk), (k, Dk), (v, Dvk)))
         ent = torch.empty((B, H, N), device=q.device, dtype=torch.float32)
         lse = torch.empty((B, H, N), device=q.device, dtype=torch.float32)
@@ -116,8 +85,6 @@ class _FlashEntropyAttention(torch.autograd.Function):
             ent[:, :, n:] = 0
             lse[:, :, n:] = 0
         ctx.save_for_backward(q, k, v, o, lse, ent)
-        ctx.sm_scale = sm_scale
-        ctx.n_valid = n
         return o, ent
 
     @staticmethod
@@ -126,6 +93,20 @@ class _FlashEntropyAttention(torch.autograd.Function):
         q, k, v, o, lse, ent = ctx.saved_tensors
         dq, dk, dv = fea_backward(q, k, v, o, lse, ent, do, de, ctx.sm_scale, ctx.n_valid)
         return dq, dk, dv, None, None, None
+
+
+def _plain_call(q, k, v):
+    """Whether flash_entropy_attention can go straight to the kernels: no gradient or transform to record (autograd's
+    function, ~12 us of host time, is then only passed through), and inputs that its forward takes as they are."""
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+        return False
+    if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    if not (type(q) is type(k) is type(v) is torch.Tensor and q.is_cuda and q.dim() == 4):
+        return False
+    D, Dv = q.shape[-1], v.shape[-1]
+    return (q.dtype in _lib.DTYPES and k.shape == q.shape and v.shape[:-1] == q.shape[:-1] and D in _HEAD_DIMS
+            and Dv in _HEAD_DIMS and not (D == 256 and Dv != 256) and _kernel_widths(D, Dv) == (D, Dv))
 
 
 def flash_entropy_attention(q, k, v, sm_scale=None, warp_specialize=True):
@@ -144,4 +125,6 @@ def flash_entropy_attention(q, k, v, sm_scale=None, warp_specialize=True):
     n = q.shape[-2]
     if sm_scale is None:
         sm_scale = q.shape[-1] ** -0.5
+    if _plain_call(q, k, v):
+        return _lib.host().fea_attention(q, k, v, sm_scale)[:2]
     return _FlashEntropyAttention.apply(q, k, v, sm_scale, n, warp_specialize)

@@ -40,60 +40,9 @@ def fea_backward_raw(q, k, v, o, lse, ent, do, de, sm_scale, dq=None, dk=None, d
     `dq_route` ("recompute" or "ds"; None lets the library choose) picks how dq is formed: a pass that
     recomputes S and dP, or a GEMM over dS^T stored by the dk / dv pass (the workspace then holds nk x nq
     16-bit values per problem)."""
-    L = _lib.lib()
-    B, H, NQ, D = q.shape
-    NK, Dv = k.shape[2], v.shape[-1] * (2 if v1 is not None else 1)
-    flags = (_lib.BWD_FOLD_K if fold_k else 0) | {None: 0, "recompute": _lib.BWD_RECOMPUTE_DQ,
-                                                   "ds": _lib.BWD_DS_DQ}[dq_route]
-    for t, name, acc_bit, f32_bit, base in ((dq, "q", _lib.BWD_ACCUM_Q, _lib.BWD_F32_Q, dq_base),
-                                            (dk, "k", _lib.BWD_ACCUM_K, _lib.BWD_F32_K, dk_base),
-                                            (dv, "v", _lib.BWD_ACCUM_V, _lib.BWD_F32_V, dv_base)):
-        if base is not None:
-            assert base.dtype == torch.float32 and (t is None or t.dtype == q.dtype), "base fp32, result q.dtype"
-            flags |= {"q": _lib.BWD_SUM_Q, "k": _lib.BWD_SUM_K, "v": _lib.BWD_SUM_V}[name]
-        elif t is not None and t.dtype != q.dtype:
-            assert t.dtype == torch.float32, "a gradient passed in must be float32 or q's dtype"
-            flags |= f32_bit if name in overwrite else acc_bit
-    if dq is None:
-        dq = torch.empty((B, H, NQ, D), device=q.device, dtype=q.dtype)
-    if dk is None:
-        dk = torch.empty((B, H, NK, D), device=q.device, dtype=q.dtype)
-    if dv is None and not (fold_k and v1 is None):
-        dv = torch.empty((B, H, NK, v1.shape[-1] if fold_k else Dv), device=q.device, dtype=q.dtype)
-    a = _lib.FeaBwdArgs()
-    a.flags = flags
-    a.dtype = _lib.DTYPES[q.dtype]
-    assert NQ % frames == 0 and NK % frames == 0
-    a.batch, a.heads, a.nq, a.nk, a.d, a.dv = B, H, NQ // frames, NK // frames, D, Dv
-    a.frames = frames
-    a.q, a.k, a.v, a.o, a.grad_o = (_lib.view(t) for t in (q, k, v, o, do))
-    a.grad_q, a.grad_k = _lib.view(dq), _lib.view(dk)
-    a.grad_v = _lib.view(dv) if dv is not None else _lib.View()
-    if dq_base is not None:
-        assert dq_base.shape == dq.shape
-        a.grad_q_base = _lib.view(dq_base)
-    if dk_base is not None:
-        assert dk_base.shape == dk.shape
-        a.grad_k_base = _lib.view(dk_base)
-    if dv_base is not None:
-        assert dv_base.shape == dv.shape
-        a.grad_v_base = _lib.view(dv_base)
-    assert lse.stride() == ent.stride() and lse.stride(2) == 1 and de.stride(2) == 1
-    a.lse, a.ent, a.grad_ent = lse.data_ptr(), ent.data_ptr(), de.data_ptr()
-    a.stat_stride_b, a.stat_stride_h = lse.stride(0), lse.stride(1)
-    a.grad_ent_stride_b, a.grad_ent_stride_h = de.stride(0), de.stride(1)
-    a.sm_scale = float(sm_scale)
-    if v1 is not None:
-        assert v1.shape == v.shape and v1.stride() == v.stride() and v1.dtype == v.dtype
-        a.v1, a.dv1 = _lib.view(v1), v1.shape[-1]
-    if delta is not None:
-        assert delta.dtype == torch.float32 and delta.stride(2) == 1
-        a.delta, a.delta_stride_b, a.delta_stride_h = delta.data_ptr(), delta.stride(0), delta.stride(1)
-    nbytes = L.vmo_fea_bwd_workspace_size(a)
-    ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-    a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
-    _lib.check(L.vmo_fea_bwd(a, _lib.stream_of(q)), "vmo_fea_bwd")
-    return dq, dk, dv
+    route = {None: 0, "recompute": _lib.BWD_RECOMPUTE_DQ, "ds": _lib.BWD_DS_DQ}[dq_route]
+    return _lib.host().fea_bwd(q, k, v, o, lse, ent, do, de, sm_scale, dq, dk, dv, overwrite, v1, fold_k, dk_base, dv_base,
+                               frames, route, dq_base, delta)
 
 
 def fea_backward(q, k, v, o, lse, ent, do, de, sm_scale, n_valid):
@@ -116,10 +65,7 @@ def fea_backward(q, k, v, o, lse, ent, do, de, sm_scale, n_valid):
     if n == N and Dk == D and Dvk == Dv:
         # no padding rows, no padded features: the kernels write the gradients once, in the memory order
         # of the caller's q, k, v (a DiT block's (B, N, H, D) buffers need no copy afterwards)
-        grads = [_lib.empty_in_layout(t, t.shape[-1], q.dtype) for t in (q, k, v)]
-        args = [_lib.row_aligned(t) for t in (q, k, v, o, do)]
-        fea_backward_raw(*args[:4], lse, ent, args[4], de, sm_scale, dq=grads[0], dk=grads[1], dv=grads[2])
-        return tuple(grads)
+        return _lib.host().fea_attention_bwd(q, k, v, o, lse, ent, do, de, sm_scale)
     dq = torch.zeros_like(q)
     dk = torch.zeros_like(k)
     dv = torch.zeros_like(v)

@@ -28,8 +28,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib
-from .kernel import fea_forward, flash_entropy_attention
-from .kernel_bwd import fea_backward_raw
+from .kernel import flash_entropy_attention
 
 # number of CUs on an MI355X; the recompute picks its split-KV count to fill them
 _NUM_CUS = 256
@@ -59,19 +58,7 @@ def _recompute_splits(problems, nq, nk):
 
 
 def _lstep_launch(q, out, ent, res, m, b, scale, last, skip, min_col_mass):
-    L = _lib.lib()
-    B, H, N, D = q.shape
-    a = _lib.LstepArgs()
-    a.dtype = _lib.DTYPES[q.dtype]
-    a.batch, a.heads, a.num_blocks, a.block_size = B, H, m, b
-    a.d = D
-    a.dv = out.shape[-1] - D if last else 0
-    a.last, a.skip_tokens = int(last), int(skip)
-    a.q, a.out, a.res = _lib.view(q), _lib.view(out), _lib.view(res)
-    a.ent = ent.data_ptr()
-    a.ent_stride_b, a.ent_stride_h = ent.stride(0), ent.stride(1)
-    a.scale, a.min_col_mass = float(scale), float(min_col_mass)
-    _lib.check(L.vmo_lstep_fwd(a, _lib.stream_of(q)), "vmo_lstep_fwd")
+    _lib.host().lstep_fwd(q, out, ent, res, m, b, scale, bool(last), skip, min_col_mass)
 
 
 def _lstep_one_tile(m, d, dv, last):
@@ -83,24 +70,8 @@ def _lstep_bwd_launch(q, out, ent, grad_res, grad_q, grad_out, m, b, scale, last
                       overwrite_q=False, delta=None):
     """Backward of one L-step (vmo_lstep_bwd): grad_q (fp32) += dL/dq (= with overwrite_q),
     grad_out = dL/d out; with `delta` ((B, H, N) fp32, one-tile grids only) also rowsum(out * grad_out)."""
-    L = _lib.lib()
-    B, H, N, D = q.shape
-    a = _lib.LstepBwdArgs()
-    a.dtype = _lib.DTYPES[q.dtype]
-    a.batch, a.heads, a.num_blocks, a.block_size = B, H, m, b
-    a.d = D
-    a.dv = out.shape[-1] - D if last else 0
-    a.last, a.skip_tokens = int(last), int(skip)
-    a.q, a.out, a.grad_res = _lib.view(q), _lib.view(out), _lib.view(grad_res)
-    a.grad_q, a.grad_out = _lib.view(grad_q), _lib.view(grad_out)
-    a.ent = ent.data_ptr()
-    a.ent_stride_b, a.ent_stride_h = ent.stride(0), ent.stride(1)
-    a.scale, a.min_col_mass = float(scale), float(min_col_mass)
-    a.flags = _lib.LSTEP_BWD_OVERWRITE_Q if overwrite_q else 0
-    if delta is not None:
-        assert delta.dtype == torch.float32 and delta.stride(2) == 1
-        a.delta, a.delta_stride_b, a.delta_stride_h = delta.data_ptr(), delta.stride(0), delta.stride(1)
-    _lib.check(L.vmo_lstep_bwd(a, _lib.stream_of(q)), "vmo_lstep_bwd")
+    _lib.host().lstep_bwd(q, out, ent, grad_res, grad_q, grad_out, m, b, scale, bool(last), skip, min_col_mass,
+                          bool(overwrite_q), delta)
 
 
 _LDS_BYTES = 160 * 1024   # per CU on gfx950
@@ -172,6 +143,7 @@ def _fused_supported(q, k, v, num_blocks):
 # "off": after the chain on the caller's stream).  Measured at cfg4 (four interleaved rounds of 100
 # steps on one box): start 1.126-1.128 ms, after_r0 1.131-1.137 ms with the same 3 key splits.
 _RECOMPUTE_OVERLAP = "start"
+_OVERLAPS = {"off": 0, "start": 1, "after_r0": 2, "after_r1": 3}
 _side_streams = {}
 
 
@@ -190,60 +162,14 @@ def _vmonarch_fused(q, k, v, m, b, num_iters, recompute_tokens, min_col_mass, st
     D ** -0.5 (q / k zero-padded past their head dim).  `qk_fp8`: the R-steps' S in fp8 (the recompute
     stays exact)."""
     B, H, N, D = q.shape
-    Dv = v.shape[-1]
     scale = D ** -0.5 if scale is None else scale
-    q, k, v = (_lib.row_aligned(t) for t in (q, k, v))
-    dev, dt = q.device, q.dtype
-    main = torch.cuda.current_stream(dev)
-    hook = stage_hook or (lambda name, phase, stream: None)
-    ent = torch.empty((B, H, N), device=dev, dtype=torch.float32)
-    z = _lib.empty_in_layout(q, Dv, dt)   # z in the caller's layout (a DiT block's (B, N, H, Dv))
     rt = min(int(recompute_tokens), N)
-    side = None
-
-    def recompute(stream):
-        # exact attention for the first rt queries (vmonarch.py:66-68), written into z
-        with torch.cuda.stream(stream):
-            hook("recompute", "begin", stream)
-            splits = _recompute_splits(B * H, rt, N)
-            fea_forward(q[:, :, :rt], k, v, None, scale, o=z[:, :, :rt], want_ent=False, want_lse=False,
-                        num_splits=splits)
-            hook("recompute", "end", stream)
-
-    def fork():
-        nonlocal side
-        side = _side_stream(dev)
-        side.wait_stream(main)   # q, k, v and z are ready on the caller's stream
-        recompute(side)
-
-    if rt > 0 and _RECOMPUTE_OVERLAP == "start":
-        fork()
-    u = None
-    for it in range(num_iters):
-        last = it == num_iters - 1
-        # R-step (vmonarch.py:50): iteration 0 folds u = q * scale into the softmax scale
-        x, s = (q, scale) if it == 0 else (u, 1.0)
-        hook(f"rstep{it}", "begin", main)
-        out, _, _ = fea_forward(x, k, k, v if last else None, s, frames=m, ent=ent, want_lse=False, qk_fp8=qk_fp8)
-        hook(f"rstep{it}", "end", main)
-        if rt > 0 and side is None and ((_RECOMPUTE_OVERLAP == "after_r0" and it == 0) or
-                                        (_RECOMPUTE_OVERLAP == "after_r1" and last)):
-            fork()
-        # L-step (vmonarch.py:51-63)
-        hook(f"lstep{it}", "begin", main)
-        if last:
-            _lstep_launch(q, out, ent, z, m, b, scale, True, rt, min_col_mass)
-        else:
-            if u is None:
-                u = torch.empty((B, H, N, D), device=dev, dtype=dt)
-            _lstep_launch(q, out, ent, u, m, b, scale, False, 0, min_col_mass)
-        hook(f"lstep{it}", "end", main)
-    if rt > 0:
-        if side is None:
-            recompute(main)
-        else:
-            main.wait_stream(side)   # z is complete on the caller's stream
-    return z
+    overlap = _OVERLAPS[_RECOMPUTE_OVERLAP] if rt > 0 else 0
+    side = _side_stream(q.device) if overlap else None
+    main = torch.cuda.current_stream(q.device) if stage_hook is not None else None
+    return _lib.host().vmonarch_fwd(q, k, v, m, b, num_iters, rt, min_col_mass, scale, qk_fp8,
+                                    _recompute_splits(B * H, rt, N) if rt > 0 else 1, overlap,
+                                    side.cuda_stream if side is not None else 0, stage_hook, main, side)
 
 
 def _hip_backward_supported(q, k, v, num_blocks):
@@ -267,117 +193,24 @@ class _VMonarchFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, m, b, num_iters, recompute_tokens, min_col_mass, scale=None):
         B, H, N, D = q.shape
-        Dv = v.shape[-1]
         scale = D ** -0.5 if scale is None else scale
-        z = _lib.empty_in_layout(q, Dv, q.dtype)
-        ctx.orders = tuple(_lib.layout_order(t) for t in (q, k, v))
-        # read in place in any memory order (the backward, like the forward, takes each head's m frames
-        # as m problems of the (B, H, m*b) tensors): no contiguous copies of a DiT block's (B, N, H, D)
-        q, k, v = (_lib.row_aligned(t) for t in (q, k, v))
-        if k.stride() != v.stride():   # the backward reads the values [k | v] as two parts with one set of strides
-            k, v = k.contiguous(), v.contiguous()
-        dev, dt = q.device, q.dtype
         rt = min(int(recompute_tokens), N)
-        saved = []
-        lse_rt = None
-        main, side = torch.cuda.current_stream(dev), None
-
-        def recompute():
-            return fea_forward(q[:, :, :rt], k, v, None, scale, o=z[:, :, :rt], want_ent=False,
-                               num_splits=_recompute_splits(B * H, rt, N))[1]
-
-        if rt > 0 and _RECOMPUTE_OVERLAP != "off":
-            # the exact recompute of rows [0, rt) beside the R/L chain, as in _vmonarch_fused (it reads q, k, v
-            # only and writes rows of z that the last L-step leaves alone)
-            side = _side_stream(dev)
-            side.wait_stream(main)
-            with torch.cuda.stream(side):
-                lse_rt = recompute()
-        u = None
-        for it in range(num_iters):
-            last = it == num_iters - 1
-            x, s = (q, scale) if it == 0 else (u, 1.0)
-            out, lse, ent = fea_forward(x, k, k, v if last else None, s, frames=m)
-            if last:
-                _lstep_launch(q, out, ent, z, m, b, scale, True, rt, min_col_mass)
-            else:
-                u = torch.empty((B, H, N, D), device=dev, dtype=dt)
-                _lstep_launch(q, out, ent, u, m, b, scale, False, 0, min_col_mass)
-            saved += [x, out, lse, ent]
-        if side is not None:
-            main.wait_stream(side)       # z and lse_rt are complete on the caller's stream
-            lse_rt.record_stream(main)   # allocated on the side stream, read by the backward on this one
-        elif rt > 0:
-            lse_rt = recompute()
+        overlap = rt > 0 and _RECOMPUTE_OVERLAP != "off"
+        ctx.orders, saved = _lib.host().vmonarch_fwd_train(
+            q, k, v, m, b, num_iters, rt, min_col_mass, scale, _recompute_splits(B * H, rt, N) if rt > 0 else 1, overlap,
+            _side_stream(q.device).cuda_stream if overlap else 0)
         ctx.dims = (m, b, num_iters, rt, float(min_col_mass), float(scale))
-        ctx.save_for_backward(q, k, v, z, lse_rt if lse_rt is not None else z.new_empty(0), *saved)
-        return z
+        ctx.save_for_backward(*saved)
+        return saved[3]
 
     @staticmethod
     def backward(ctx, dz):
         m, b, num_iters, rt, min_col_mass, scale = ctx.dims
-        q, k, v, z, lse_rt, *saved = ctx.saved_tensors
-        B, H, N, D = q.shape
-        Dv = v.shape[-1]
-        dev, dt = q.device, q.dtype
-        dz = _lib.row_aligned(dz.to(dt))
-        f32 = torch.float32
-        # Call order: the L- and R-step backwards from the last iteration down, R-step 0's last of all and the
-        # recompute's (rows [0, rt), vmonarch.py:66-68) just before it.  Every gradient is written once, in
-        # the caller's dtype and memory order, by the last call that contributes to it: the fp32 sum of the
-        # earlier contributions plus its own (VMO_BWD_SUM_*), so no conversion pass follows.  dq: the
-        # L-steps (the first overwrites, the rest add), the recompute, then R-step 0 (x = q).  dk: every
-        # R-step (values start with k: the kernels fold k's value-role gradient into dk, as autograd's sum
-        # over k's uses at vmonarch.py:50 does), the recompute, R-step 0 last.  dv: the last R-step (values
-        # [k | v]) and the recompute.
-        gq, gk, gv = (_lib.empty_in_order(o, (B, H, N), f, dt, dev) for o, f in zip(ctx.orders, (D, D, Dv)))
-        dq = torch.empty((B, H, N, D), device=dev, dtype=f32)
-        partial = {"k": torch.empty((B, H, N, D), device=dev, dtype=f32),
-                   "v": torch.empty((B, H, N, Dv), device=dev, dtype=f32)}
-        started = {"k": False, "v": False}
-        final = {"k": gk, "v": gv}
-        v_writers = ([num_iters - 1] if num_iters > 1 else []) + (["rt"] if rt > 0 else []) + ([0] if num_iters == 1 else [])
-
-        def grad_args(x, last_writer):
-            """fea_backward_raw arguments for gradient x ("k" or "v") of one call: into the fp32 partial sum
-            (overwriting it on the first call), or, from its last writer, into the dtype result."""
-            if last_writer:
-                return ({f"d{x}": final[x], f"d{x}_base": partial[x]} if started[x] else {f"d{x}": final[x]}), ""
-            first = not started[x]
-            started[x] = True
-            return {f"d{x}": partial[x]}, (x if first else "")
-
-        de = torch.zeros((B, H, N), device=dev, dtype=f32)
-        # rowsum(out * d out), formed by the L-step backward that writes d out (one-tile grids), read by the
-        # R-step backward in place of another pass over both
-        delta = torch.empty((B, H, N), device=dev, dtype=f32) if _lstep_one_tile(m, D, Dv, True) else None
-        g = dz
-        for it in reversed(range(num_iters)):
-            last = it == num_iters - 1
-            x, out, lse, ent = saved[4 * it: 4 * it + 4]
-            dout = torch.empty_like(out)
-            _lstep_bwd_launch(q, out, ent, g, dq, dout, m, b, scale, last, rt if last else 0, min_col_mass,
-                              overwrite_q=last, delta=delta)
-            if it == 0 and rt > 0:
-                # the exact attention of the first rt queries; it reads every key and value
-                zeros = torch.zeros((B, H, rt), device=dev, dtype=f32)
-                kw, ow = grad_args("k", False)
-                kv, ov = grad_args("v", v_writers[-1] == "rt")
-                fea_backward_raw(q[:, :, :rt], k, v, z[:, :, :rt], lse_rt, zeros, _lib.row_aligned(dz[:, :, :rt]), zeros,
-                                 scale, dq=dq[:, :, :rt], overwrite=ow + ov, **kw, **kv)
-            # values k, or [k | v] read from the two tensors in place (vmonarch.py:50); m frames per head
-            kw, ow = grad_args("k", it == 0)
-            if last:
-                kv, ov = grad_args("v", v_writers[-1] == it)
-                kw.update(kv)
-                ow += ov
-            if it == 0:   # R-step 0 reads q itself: dq's last contribution
-                kw.update(dq=gq, dq_base=dq)
-            gx, _, _ = fea_backward_raw(x, k, k, out, lse, ent, dout, de, scale if it == 0 else 1.0, overwrite=ow,
-                                        v1=v if last else None, fold_k=True, frames=m, delta=delta, **kw)
-            if it > 0:
-                g = gx                      # dL/du of the previous L-step's output
-        return gq, gk, gv, None, None, None, None, None, None
+        saved = ctx.saved_tensors
+        D, Dv = saved[0].shape[-1], saved[2].shape[-1]
+        grads = _lib.host().vmonarch_bwd(ctx.orders, saved, dz, m, b, num_iters, rt, min_col_mass, scale,
+                                         _lstep_one_tile(m, D, Dv, True))
+        return *grads, None, None, None, None, None, None
 
 
 def _vmonarch_composed(q, k, v, num_blocks, block_size, num_iters, recompute_tokens, min_col_mass):
