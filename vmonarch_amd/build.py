@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libvmonarch_gfx950.so")
-SOURCES = ["capi.hip", "fea_fwd.hip", "fea_bwd.hip", "lstep.hip", "lstep_mb.hip"]
+SOURCES = ["capi.hip", "fea_fwd.hip", "fea_fwd_ks.hip", "fea_bwd.hip", "lstep.hip", "lstep_mb.hip"]
 HOST_LIB = os.path.join(HERE, "_vmo_host.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
