@@ -7,8 +7,8 @@ B=1, H=12, N=32760, D=128 bf16; q, k ~ 0.5 N(0,1), v ~ N(0,1) from seed 0, resid
 One step = one full forward (2 R-steps, 2 L-steps, the exact recompute).
 
 Prints ONE JSON line.  `value` is algorithmic TFLOP/s of the whole forward (1107.43 GFLOP / step,
-padding and softmax excluded) in the production launch order, where the exact recompute runs on a
-second stream beside the R/L chain.  `roofline` is the dominant kernel (the flash-entropy R-step
+padding and softmax excluded) in the production launch order, the exact recompute placed where the
+library puts it by default (in one launch with R-step 0).  `roofline` is the dominant kernel (the flash-entropy R-step
 launch with values [k | v]) and `kernels` every launch, timed with HIP events on the launch stream
 inside a second timed region that runs the same launches serially (each alone on the GPU);
 `ms_per_step_serial` is that region's step time.  `graph_replay` checks that the production-order step
@@ -274,7 +274,7 @@ def main():
 
     # One step = VMonarchAttention.forward; without autograd that is exactly _vmonarch_fused (checked
     # bit for bit below).  Two timed regions of `steps` steps each:
-    #  * the production order (the exact recompute on a second stream beside the R/L chain): `value`;
+    #  * the production order (the exact recompute where the library puts it by default): `value`;
     #  * the serial order (every launch alone on one stream) with an event before and after each
     #    launch group on its stream: the per-launch breakdown and `roofline` (a launch that shares the
     #    GPU with another has no meaningful rate of its own).

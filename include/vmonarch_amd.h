@@ -270,6 +270,15 @@ size_t vmo_fea_fwd_workspace_size(const vmo_fea_fwd_args* args);
 int vmo_fea_fwd(const vmo_fea_fwd_args* args, void* stream);
 
 /*
+ * Two independent forwards, a and b, issued together: results as vmo_fea_fwd(a) and vmo_fea_fwd(b) (neither may
+ * read what the other writes).  VMonarch's exact recompute (a: values v, no entropy, any number of splits) and an
+ * R-step with values k (b: w0 aliasing k, entropy, one split) of the same dtype and d = dw0 in {64, 128} run in one
+ * launch, side by side without a second stream; any other two run one after the other.  No counterpart in the
+ * reference.  Both are checked before any launch.
+ */
+int vmo_fea_fwd_pair(const vmo_fea_fwd_args* a, const vmo_fea_fwd_args* b, void* stream);
+
+/*
  * Allocation-free variant of vmo_fea_fwd.  No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  Same arguments and results as vmo_fea_fwd, except that `workspace` /

@@ -39,8 +39,9 @@ constexpr int fwd_min_blocks() {
   return (D >= 256 || DW0 >= 256 || (ENT == kEntOnline && tile_w(D) < DW0) || (DW1 > 0 && DW1 < D)) ? 1 : 8 / WAVES;
 }
 
+// One workgroup's tile, logical index L.
 template <bool F16, int D, int DW0, int DW1, bool W0K, int ENT, bool SPLIT, int WAVES, bool QK8>
-__global__ __launch_bounds__(64 * WAVES, (fwd_min_blocks<D, DW0, DW1, ENT, WAVES>())) void fea_fwd_kernel(FwdParams p) {
+__device__ __forceinline__ void fea_fwd_tile(const FwdParams& p, const int L) {
   using E = Elem<F16>;
   using T = typename E::T;
   using V8 = typename E::V8;
@@ -72,11 +73,6 @@ __global__ __launch_bounds__(64 * WAVES, (fwd_min_blocks<D, DW0, DW1, ENT, WAVES
   VMO_LDS char* smem = (VMO_LDS char*)smem_raw;
   const uint32_t smem_u32 = (uint32_t)(uintptr_t)smem;
 
-  // XCD-aware block -> tile map: block b runs on XCD b % 8, so give each XCD a contiguous run of
-  // logical tiles (all query tiles of a problem then share one L2 for their K / W traffic).
-  const int per_xcd = gridDim.x >> 3;
-  const int L = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (L >= p.total_wg) return;
   // Integer division runs on the vector unit; readfirstlane brings the uniform results back to
   // scalar registers, so the per-tile address arithmetic stays scalar.  The variants with eight
   // accumulator blocks are short of registers: for them the extra scalar values cost more (their
@@ -646,6 +642,30 @@ __global__ __launch_bounds__(64 * WAVES, (fwd_min_blocks<D, DW0, DW1, ENT, WAVES
   }
 }
 
+// XCD-aware block -> tile map: block b runs on XCD b % 8, so give each XCD a contiguous run of
+// logical tiles (all query tiles of a problem then share one L2 for their K / W traffic).
+__device__ __forceinline__ int fwd_logical(int block, int grid) { return (block & 7) * (grid >> 3) + (block >> 3); }
+
+template <bool F16, int D, int DW0, int DW1, bool W0K, int ENT, bool SPLIT, int WAVES, bool QK8>
+__global__ __launch_bounds__(64 * WAVES, (fwd_min_blocks<D, DW0, DW1, ENT, WAVES>())) void fea_fwd_kernel(FwdParams p) {
+  const int L = fwd_logical(blockIdx.x, gridDim.x);
+  if (L < p.total_wg) fea_fwd_tile<F16, D, DW0, DW1, W0K, ENT, SPLIT, WAVES, QK8>(p, L);
+}
+
+// Two independent launches in one grid: blocks below grid_a run the exact recompute of VMonarch (a: values v, no
+// entropy, one key range or several), the others an R-step with values k (b).
+template <bool F16, int D, bool SPLIT>
+__global__ __launch_bounds__(64 * kFwdWavesSmall, 2) void fea_fwd_pair_kernel(FwdParams a, FwdParams b, int grid_a) {
+  const int blk = blockIdx.x;
+  if (blk < grid_a) {
+    const int L = fwd_logical(blk, grid_a);
+    if (L < a.total_wg) fea_fwd_tile<F16, D, D, 0, false, kEntNone, SPLIT, kFwdWavesSmall, false>(a, L);
+  } else {
+    const int L = fwd_logical(blk - grid_a, (int)gridDim.x - grid_a);
+    if (L < b.total_wg) fea_fwd_tile<F16, D, D, 0, true, kEntFromPK, false, kFwdWavesSmall, false>(b, L);
+  }
+}
+
 // Merge split-KV partials: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M).
 template <bool F16, int DWT>
 __global__ __launch_bounds__(256) void fea_combine_kernel(FwdParams p) {
@@ -751,6 +771,27 @@ static int launch_fwd(FwdParams p, hipStream_t stream) {
   constexpr int DWT = DW0 + DW1;
   const int64_t threads = (int64_t)p.problems * p.nq * (DWT / 4);
   hipLaunchKernelGGL((fea_combine_kernel<F16, DWT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p);
+  return launch_status("fea_combine");
+}
+
+// The pair kernel for a (the recompute) and b (an R-step with values k), then the merge of a's key splits.
+template <bool F16, int D, bool SPLIT>
+static int launch_pair(FwdParams a, FwdParams b, hipStream_t stream) {
+  constexpr int SA = fwd_stage_bytes<D, D, 0, false, false>(), SB = fwd_stage_bytes<D, D, 0, true, false>();
+  constexpr int LA = fwd_slots(SA, kFwdWavesSmall) * SA, LB = fwd_slots(SB, kFwdWavesSmall) * SB, LDS = LA > LB ? LA : LB;
+  static_assert(LDS <= 65536 && LDS >= kFwdWavesSmall * kEpiPatchBytes, "LDS within the default limit");
+  constexpr int BM = 32 * kFwdQB * kFwdWavesSmall;
+  for (FwdParams* p : {&a, &b}) {
+    p->q_tiles = (p->nq + BM - 1) / BM;
+    p->total_wg = p->problems * p->splits * p->q_tiles;
+  }
+  const int grid_a = xcd_grid(a.total_wg), grid_b = xcd_grid(b.total_wg);
+  hipLaunchKernelGGL((fea_fwd_pair_kernel<F16, D, SPLIT>), dim3(grid_a + grid_b), dim3(64 * kFwdWavesSmall), LDS, stream, a, b,
+                     grid_a);
+  const int rc = launch_status("fea_fwd_pair");
+  if (rc != VMO_OK || !SPLIT) return rc;
+  const int64_t threads = (int64_t)a.problems * a.nq * (D / 4);
+  hipLaunchKernelGGL((fea_combine_kernel<F16, D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a);
   return launch_status("fea_combine");
 }
 
@@ -864,15 +905,25 @@ extern "C" size_t vmo_fea_fwd_workspace_size(const vmo_fea_fwd_args* a) {
 
 namespace vmo {
 
-// The forward behind both entry points: `workspace` / `workspace_bytes` hold the split-KV partials (the
-// caller's for vmo_fea_fwd, the library's static scratch for vmo_fea_fwd_noalloc).
-static int fea_fwd_impl(const vmo_fea_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+// Checks the arguments and fills the launch parameters (*empty: nothing to launch).  `workspace` /
+// `workspace_bytes` hold the split-KV partials (the caller's, or the library's static scratch for
+// vmo_fea_fwd_noalloc).
+struct FwdLaunch {
+  FwdParams p;
+  bool f16, w0k, ent, split, qk8, empty;
+  int d, dw0, dw1;
+};
+static int fea_fwd_prepare(const vmo_fea_fwd_args* a, void* workspace, size_t workspace_bytes, FwdLaunch* out) {
+  out->empty = false;
   if (!a) return set_error(VMO_ERR_INVALID, "fea_fwd: null args");
   if (a->dtype != VMO_DTYPE_BF16 && a->dtype != VMO_DTYPE_F16)
     return set_error(VMO_ERR_INVALID, "fea_fwd: dtype %d", a->dtype);
   if (a->batch < 0 || a->heads < 0 || a->frames < 0 || a->nq < 0 || a->nk < 0)
     return set_error(VMO_ERR_INVALID, "fea_fwd: negative size");
-  if ((int64_t)a->batch * a->heads * a->frames * a->nq == 0) return VMO_OK;
+  if ((int64_t)a->batch * a->heads * a->frames * a->nq == 0) {
+    out->empty = true;
+    return VMO_OK;
+  }
   if (a->nk == 0) return set_error(VMO_ERR_INVALID, "fea_fwd: no keys");
   if (!(a->sm_scale >= 0.f) || a->sm_scale > 3.0e38f)
     return set_error(VMO_ERR_INVALID, "fea_fwd: sm_scale must be finite and >= 0");
@@ -924,10 +975,31 @@ static int fea_fwd_impl(const vmo_fea_fwd_args* a, void* workspace, size_t works
     p.k8_tiles = (a->nk + kFwdBN - 1) / kFwdBN;
     p.k8_scale = (float*)((char*)p.k8 + (problems * a->nk * a->d + 255) / 256 * 256);
   }
-  hipStream_t s = (hipStream_t)stream;
-  const bool qk8 = a->qk_fp8 != 0;
-  if (a->dtype == VMO_DTYPE_F16) return dispatch_fwd<true>(p, a->d, a->dw0, a->dw1, w0k, ent, splits > 1, qk8, s);
-  return dispatch_fwd<false>(p, a->d, a->dw0, a->dw1, w0k, ent, splits > 1, qk8, s);
+  *out = FwdLaunch{p, a->dtype == VMO_DTYPE_F16, w0k, ent, splits > 1, a->qk_fp8 != 0, false, a->d, a->dw0, a->dw1};
+  return VMO_OK;
+}
+
+static int fea_fwd_launch(const FwdLaunch& l, hipStream_t s) {
+  if (l.empty) return VMO_OK;
+  return l.f16 ? dispatch_fwd<true>(l.p, l.d, l.dw0, l.dw1, l.w0k, l.ent, l.split, l.qk8, s)
+               : dispatch_fwd<false>(l.p, l.d, l.dw0, l.dw1, l.w0k, l.ent, l.split, l.qk8, s);
+}
+
+static int fea_fwd_impl(const vmo_fea_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+  FwdLaunch l;
+  const int rc = fea_fwd_prepare(a, workspace, workspace_bytes, &l);
+  return rc != VMO_OK ? rc : fea_fwd_launch(l, (hipStream_t)stream);
+}
+
+// Whether a and b are what the pair kernel is built for (see fea_fwd_pair_kernel).
+static bool pair_built(const FwdLaunch& a, const FwdLaunch& b) {
+  return !a.empty && !b.empty && a.f16 == b.f16 && a.d == b.d && (a.d == 64 || a.d == 128) && a.dw0 == a.d && b.dw0 == b.d &&
+         a.dw1 == 0 && b.dw1 == 0 && !a.ent && !a.w0k && b.ent && b.w0k && !b.split && !a.qk8 && !b.qk8;
+}
+template <bool F16>
+static int dispatch_pair(const FwdLaunch& a, const FwdLaunch& b, hipStream_t s) {
+  if (a.d == 64) return a.split ? launch_pair<F16, 64, true>(a.p, b.p, s) : launch_pair<F16, 64, false>(a.p, b.p, s);
+  return a.split ? launch_pair<F16, 128, true>(a.p, b.p, s) : launch_pair<F16, 128, false>(a.p, b.p, s);
 }
 
 // Scratch of the allocation-free entry point: split-KV partials (fp32 o and lse of every split), fully
@@ -963,6 +1035,20 @@ static int scratch_on_current_device(void** out) {
 extern "C" int vmo_fea_fwd(const vmo_fea_fwd_args* a, void* stream) {
   vmo::clear_error();
   return vmo::fea_fwd_impl(a, a ? a->workspace : nullptr, a ? a->workspace_bytes : 0, stream);
+}
+
+extern "C" int vmo_fea_fwd_pair(const vmo_fea_fwd_args* a, const vmo_fea_fwd_args* b, void* stream) {
+  using namespace vmo;
+  clear_error();
+  FwdLaunch la, lb;
+  int rc = fea_fwd_prepare(a, a ? a->workspace : nullptr, a ? a->workspace_bytes : 0, &la);
+  if (rc != VMO_OK) return rc;
+  rc = fea_fwd_prepare(b, b ? b->workspace : nullptr, b ? b->workspace_bytes : 0, &lb);
+  if (rc != VMO_OK) return rc;
+  const hipStream_t s = (hipStream_t)stream;
+  if (pair_built(la, lb)) return la.f16 ? dispatch_pair<true>(la, lb, s) : dispatch_pair<false>(la, lb, s);
+  rc = fea_fwd_launch(la, s);
+  return rc != VMO_OK ? rc : fea_fwd_launch(lb, s);
 }
 
 extern "C" int vmo_fea_fwd_noalloc(const vmo_fea_fwd_args* a, void* stream) {

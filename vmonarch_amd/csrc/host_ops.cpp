@@ -144,6 +144,21 @@ Tensor run_fwd(const FwdCall& c, void* stream) {
   check(vmo_fea_fwd(&a, stream), "vmo_fea_fwd");
   return ws;
 }
+// a and b together (vmo_fea_fwd_pair) on the current stream
+void run_pair(const FwdCall& ca, const FwdCall& cb, void* stream) {
+  vmo_fea_fwd_args a = fwd_args(ca), b = fwd_args(cb);
+  Tensor wa, wb;
+  auto reserve = [&](vmo_fea_fwd_args& x, Tensor& ws) {
+    if (const size_t bytes = vmo_fea_fwd_workspace_size(&x)) {
+      ws = workspace(bytes, ca.q);
+      x.workspace = ws.data_ptr();
+      x.workspace_bytes = bytes;
+    }
+  };
+  reserve(a, wa);
+  reserve(b, wb);
+  check(vmo_fea_fwd_pair(&a, &b, stream), "vmo_fea_fwd_pair");
+}
 const Tensor* ptr(const OptT& t) { return t ? &*t : nullptr; }
 
 std::tuple<Tensor, OptT, OptT> fea_fwd(const Tensor& q, const Tensor& k, const Tensor& w0, const OptT& w1, double sm_scale,
@@ -319,9 +334,9 @@ struct SideStream {
   }
 };
 
-// Where the recompute runs: on the caller's stream after the chain, or on the side stream, forked at the start,
-// after R-step 0 or after the last R-step.
-enum Overlap { kOff = 0, kStart = 1, kAfterR0 = 2, kAfterR1 = 3 };
+// Where the recompute runs: on the caller's stream after the chain; on the side stream, forked at the start, after
+// R-step 0 or after the last R-step; or in one launch with R-step 0 (with more than one iteration: its values are k).
+enum Overlap { kOff = 0, kStart = 1, kAfterR0 = 2, kAfterR1 = 3, kWithR0 = 4 };
 
 struct Stages {   // the caller's stage hook (None: none), with the torch stream objects it is told of
   py::object hook, main, side;
@@ -343,9 +358,11 @@ Tensor vmonarch_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, int64_
   Tensor ws;                           // the recompute's workspace: held until its stream is joined
   SideStream ss(main, side_handle);
   // exact attention of the first rt queries, into rows of z that the L-steps do not write
+  const FwdCall exact_rows{q, k, v, nullptr, scale, 1, z, nullptr, nullptr, splits, false, rt};
+  const bool with_r0 = rt > 0 && iters > 1 && overlap == kWithR0;
   auto recompute = [&](void* stream, bool on_side) {
     stage("recompute", -1, "begin", on_side);
-    ws = run_fwd({q, k, v, nullptr, scale, 1, z, nullptr, nullptr, splits, false, rt}, stream);
+    ws = run_fwd(exact_rows, stream);
     stage("recompute", -1, "end", on_side);
   };
   bool forked = false;
@@ -360,7 +377,9 @@ Tensor vmonarch_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, int64_
     const bool last = it == iters - 1;
     out = at::empty({B, H, N, D + (last ? Dv : 0)}, q.options());
     stage("rstep", it, "begin");   // iteration 0 folds u = q * scale into the softmax scale
-    run_fwd({it == 0 ? q : u, k, k, last ? &v : nullptr, it == 0 ? scale : 1.0, m, out, nullptr, &ent, 1, qk_fp8, -1}, main);
+    const FwdCall rstep{it == 0 ? q : u, k, k, last ? &v : nullptr, it == 0 ? scale : 1.0, m, out, nullptr, &ent, 1, qk_fp8, -1};
+    if (with_r0 && it == 0) run_pair(exact_rows, rstep, main);
+    else run_fwd(rstep, main);
     stage("rstep", it, "end");
     if (rt > 0 && !forked && ((overlap == kAfterR0 && it == 0) || (overlap == kAfterR1 && last))) fork();
     stage("lstep", it, "begin");
@@ -372,7 +391,7 @@ Tensor vmonarch_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, int64_
     }
     stage("lstep", it, "end");
   }
-  if (rt > 0) {
+  if (rt > 0 && !with_r0) {
     if (forked) ss.join();   // z is complete on the caller's stream
     else recompute(main, false);
   }
@@ -383,7 +402,7 @@ Tensor vmonarch_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, int64_
 std::tuple<std::vector<int>, std::vector<Tensor>> vmonarch_fwd_train(const Tensor& q0, const Tensor& k0, const Tensor& v0,
                                                                      int64_t m, int64_t b, int64_t iters, int64_t rt,
                                                                      double min_col_mass, double scale, int64_t splits,
-                                                                     bool overlap, int64_t side_handle) {
+                                                                     int overlap, int64_t side_handle) {
   std::vector<int> orders;
   for (const Tensor* t : {&q0, &k0, &v0})
     for (int d : layout_order(*t)) orders.push_back(d);
@@ -399,12 +418,11 @@ std::tuple<std::vector<int>, std::vector<Tensor>> vmonarch_fwd_train(const Tenso
   Tensor lse_rt, ws;
   SideStream ss(main, side_handle);
   if (rt > 0) lse_rt = at::empty({B, H, rt}, f32(q));
-  auto recompute = [&](void* stream) {
-    ws = run_fwd({q, k, v, nullptr, scale, 1, z, &lse_rt, nullptr, splits, false, rt}, stream);
-  };
-  if (rt > 0 && overlap) {
+  const FwdCall exact_rows{q, k, v, nullptr, scale, 1, z, &lse_rt, nullptr, splits, false, rt};
+  const bool with_r0 = rt > 0 && iters > 1 && overlap == kWithR0, forked = rt > 0 && overlap != kOff && overlap != kWithR0;
+  if (forked) {
     ss.fork();
-    recompute((void*)ss.side);
+    ws = run_fwd(exact_rows, (void*)ss.side);
   }
   std::vector<Tensor> saved;
   Tensor u;
@@ -413,7 +431,9 @@ std::tuple<std::vector<int>, std::vector<Tensor>> vmonarch_fwd_train(const Tenso
     Tensor out = at::empty({B, H, N, D + (last ? Dv : 0)}, q.options());
     Tensor lse = at::empty({B, H, N}, f32(q)), ent = at::empty({B, H, N}, f32(q));
     const Tensor x = it == 0 ? q : u;
-    run_fwd({x, k, k, last ? &v : nullptr, it == 0 ? scale : 1.0, m, out, &lse, &ent, 1, false, -1}, main);
+    const FwdCall rstep{x, k, k, last ? &v : nullptr, it == 0 ? scale : 1.0, m, out, &lse, &ent, 1, false, -1};
+    if (with_r0 && it == 0) run_pair(exact_rows, rstep, main);
+    else run_fwd(rstep, main);
     if (last) {
       lstep_fwd(q, out, ent, z, m, b, scale, true, rt, min_col_mass);
     } else {
@@ -422,10 +442,8 @@ std::tuple<std::vector<int>, std::vector<Tensor>> vmonarch_fwd_train(const Tenso
     }
     for (const Tensor& t : {x, out, lse, ent}) saved.push_back(t);
   }
-  if (rt > 0) {
-    if (overlap) ss.join();   // z and lse_rt are complete on the caller's stream
-    else recompute(main);
-  }
+  if (forked) ss.join();   // z and lse_rt are complete on the caller's stream
+  else if (rt > 0 && !with_r0) run_fwd(exact_rows, main);
   std::vector<Tensor> all{q, k, v, z, rt > 0 ? lse_rt : at::empty({0}, q.options())};
   all.insert(all.end(), saved.begin(), saved.end());
   return {orders, all};

@@ -47,14 +47,33 @@ def _row_block_attention(x, k, w):
 _ROW_BLOCK_ATTENTION = _row_block_attention   # the seam as shipped; patched seams use the composed path
 
 
-def _recompute_splits(problems, nq, nk):
-    """Key splits of the recompute: the fewest that fill ~80% of one round of workgroup slots (two 128-query
-    workgroups per CU), each split keeping >= 512 keys.  Fewer splits write fewer fp32 partials; a split count
-    whose workgroups spill a little into another round leaves that round mostly idle (measured at cfg4, 156
-    query tiles: 3 splits 0.300 ms, 8 splits 0.309 ms, 16 splits 0.336 ms)."""
+def _recompute_splits(problems, nq, nk, paired=False):
+    """Key splits of the recompute, each merged from fp32 partials by one more launch.
+
+    On its own: the fewest that fill ~80% of one round of workgroup slots (two 128-query workgroups per CU), each
+    split keeping >= 512 keys (measured at cfg4, 156 query tiles: 3 splits 0.300 ms, 8 splits 0.309, 16 splits 0.336).
+    In one launch with R-step 0, whose workgroups fill the other slots: the fewest that make 120 workgroups, at least
+    two (one workgroup walking all keys would outlast the R-step) and at most eight, each of >= 256 keys.  Measured,
+    whole forward in us at 2 / 4 / 8 / 16 splits: 16 query tiles x 4096 keys 75.9 / 64.6 / 61.0 / 65.4; 24 x 4200 88.2 /
+    76.1 / 81.9 / 85.1; 48 x 13200 279 / 255 / 261 / 271; 156 x 32760 1209 / 1215 / 1237 / 1269 (1 split: 1236)."""
     base = problems * ((nq + 127) // 128)
+    if paired:
+        return max(1, min(8, max(2, -(-120 // base)), nk // 256))
     want = -(-int(0.8 * 2 * _NUM_CUS) // base)
     return max(1, min(16, want, nk // 512))
+
+
+def _recompute_plan(B, H, N, D, Dv, num_iters, rt):
+    """(order, key splits) of the exact recompute of the first rt queries; see _RECOMPUTE_OVERLAP."""
+    order = _RECOMPUTE_OVERLAP
+    if rt <= 0:
+        return 0, 1
+    if order == "auto":
+        if num_iters > 1 and D == Dv and D in (64, 128):
+            order = "with_r0"
+        else:
+            order = "start" if 2.0 * B * H * rt * N * (D + Dv) >= _FORK_MIN_FLOPS else "off"
+    return _OVERLAPS[order], _recompute_splits(B * H, rt, N, order == "with_r0")
 
 
 def _lstep_launch(q, out, ent, res, m, b, scale, last, skip, min_col_mass):
@@ -137,13 +156,18 @@ def _fused_supported(q, k, v, num_blocks):
             and k.shape == q.shape and v.shape[:-1] == q.shape[:-1])
 
 
-# Where the exact recompute of the first rt queries starts on its own stream: it reads q, k, v only
-# and writes rows [0, rt) of z, which the L-steps never write, so it can run beside the R/L chain
-# ("start": with R-step 0, "after_r0": beside L-step 0 onwards, "after_r1": beside the last L-step,
-# "off": after the chain on the caller's stream).  Measured at cfg4 (four interleaved rounds of 100
-# steps on one box): start 1.126-1.128 ms, after_r0 1.131-1.137 ms with the same 3 key splits.
-_RECOMPUTE_OVERLAP = "start"
-_OVERLAPS = {"off": 0, "start": 1, "after_r0": 2, "after_r1": 3}
+# Where the exact recompute of the first rt queries runs: it reads q, k, v only and writes rows [0, rt) of z, which
+# the L-steps never write, so it can run beside the R/L chain.  "with_r0": its workgroups in one launch with R-step
+# 0's; "start" / "after_r0" / "after_r1": on a second stream, forked there and joined at the end; "off": after the
+# chain; "auto": with_r0 where that launch is built (more than one iteration, equal head dims of 64 or 128),
+# otherwise start from _FORK_MIN_FLOPS on, else off.  Fork and join cost ~45 us of host time in the HIP runtime
+# (event records and cross-stream waits), which small calls waited for; the shared launch costs none.  Whole
+# forward, us, start / off / with_r0: 4 x 64 grid, 2 heads 59.8 / 25.7 / 21.2; 16 x 256, 8 problems 66.8 / 67.4 / 57.7;
+# 21 x 400, 12 heads 150.6 / 157.1 / 151.4; 21 x 800 386.8 / 389.9 / 380.3; 33 x 993 902 / 909 / 889; 21 x 1560
+# 1181 / 1194 / 1176.
+_RECOMPUTE_OVERLAP = "auto"
+_FORK_MIN_FLOPS = 4e9   # (~the same figures: 16 x 256, 4.3 GFLOP of exact rows, start and off are level)
+_OVERLAPS = {"off": 0, "start": 1, "after_r0": 2, "after_r1": 3, "with_r0": 4}
 _side_streams = {}
 
 
@@ -164,11 +188,10 @@ def _vmonarch_fused(q, k, v, m, b, num_iters, recompute_tokens, min_col_mass, st
     B, H, N, D = q.shape
     scale = D ** -0.5 if scale is None else scale
     rt = min(int(recompute_tokens), N)
-    overlap = _OVERLAPS[_RECOMPUTE_OVERLAP] if rt > 0 else 0
-    side = _side_stream(q.device) if overlap else None
+    overlap, splits = _recompute_plan(B, H, N, D, v.shape[-1], num_iters, rt)
+    side = _side_stream(q.device) if overlap not in (0, 4) else None
     main = torch.cuda.current_stream(q.device) if stage_hook is not None else None
-    return _lib.host().vmonarch_fwd(q, k, v, m, b, num_iters, rt, min_col_mass, scale, qk_fp8,
-                                    _recompute_splits(B * H, rt, N) if rt > 0 else 1, overlap,
+    return _lib.host().vmonarch_fwd(q, k, v, m, b, num_iters, rt, min_col_mass, scale, qk_fp8, splits, overlap,
                                     side.cuda_stream if side is not None else 0, stage_hook, main, side)
 
 
@@ -195,10 +218,10 @@ class _VMonarchFunction(torch.autograd.Function):
         B, H, N, D = q.shape
         scale = D ** -0.5 if scale is None else scale
         rt = min(int(recompute_tokens), N)
-        overlap = rt > 0 and _RECOMPUTE_OVERLAP != "off"
+        overlap, splits = _recompute_plan(B, H, N, D, v.shape[-1], num_iters, rt)
         ctx.orders, saved = _lib.host().vmonarch_fwd_train(
-            q, k, v, m, b, num_iters, rt, min_col_mass, scale, _recompute_splits(B * H, rt, N) if rt > 0 else 1, overlap,
-            _side_stream(q.device).cuda_stream if overlap else 0)
+            q, k, v, m, b, num_iters, rt, min_col_mass, scale, splits, overlap,
+            _side_stream(q.device).cuda_stream if overlap not in (0, 4) else 0)
         ctx.dims = (m, b, num_iters, rt, float(min_col_mass), float(scale))
         ctx.save_for_backward(*saved)
         return saved[3]
