@@ -45,7 +45,7 @@ constexpr int kMbMaxFrames = 32 * kMbMaxBlocks;  // m <= 128
 // workgroup fits either way, and the whole patches store faster.
 __host__ __device__ constexpr int mb_bwd_patch_rows(bool last, int M) { return last && M <= 64 ? 16 : 32; }
 struct MbLayout {
-  int q, k, y, g, e, lse, part, rs, f, dc, patch, total;
+  int q, k, y, g, e, lse, part, rs, f, dc, patch, patch_rows, mat0, mat1, total;
 };
 // A staged tile holds M = 32 ceil(m / 32) rows, those past m zeros (finite data whose weights are exact zeros).
 // A compact tile (CT: the two-block last-step kernels up to kMbCompactMaxFrames, where it lets one more column
@@ -70,7 +70,7 @@ __device__ __forceinline__ int mb_phys_row(int r, int m) {
 }
 
 __host__ __device__ inline MbLayout mb_layout(int m, int d, int dv, bool last, bool bwd, bool compact) {
-  MbLayout L;
+  MbLayout L{};
   const int M = 32 * ((m + 31) / 32);
   int off = 0;
   auto take = [&](int bytes) { const int o = off; off += (bytes + 255) / 256 * 256; return o; };
@@ -85,8 +85,52 @@ __host__ __device__ inline MbLayout mb_layout(int m, int d, int dv, bool last, b
   L.f = bwd ? take(M * 4) : 0;
   L.dc = bwd ? take(M * 4) : 0;
   L.patch = bwd ? take(kMbWaves * mb_bwd_patch_rows(last, M) * 32 * 4) : 0;
+  L.patch_rows = mb_bwd_patch_rows(last, M);
   L.total = off > kMbWaves * kEpiPatchBytes ? off : kMbWaves * kEpiPatchBytes;
   return L;
+}
+
+// The one-block-per-wave backward (every grid that is not two blocks on four waves) hands m x m matrices -- the
+// attention, dl, a f, rounded to the 16-bit type as MFMA operands -- from the waves that form them (one row or column
+// block each) to the waves that need them in the other orientation, through an LDS matrix of M rows of 256 bytes (M
+// <= 128 columns).  It overlays what is dead by then: the last step's kr and y tiles, the other steps' q tile and the
+// row-store patches after it.  The last step reads its waves' own q and g rows from HBM into registers (MFMA operands)
+// and writes their tiles from there, where the other orientation needs them whole, beside the matrix; so kr and y are
+// all it stages, and two columns share a CU up to 128 frames at 128-wide heads.  The patches hold 32, 16 or 8 rows
+// per wave: the most that does not cost a column per CU.
+constexpr int kMbMatRow = 256;
+__host__ __device__ inline MbLayout mb_layout_bwd1(int m, int d, int dv, bool last) {
+  const int M = 32 * ((m + 31) / 32), mat = M * kMbMatRow;
+  MbLayout best{};
+  for (int rows = 32; rows >= 8; rows /= 2) {
+    MbLayout L{};
+    int off = 0;
+    auto take = [&](int bytes) { const int o = off; off += (bytes + 255) / 256 * 256; return o; };
+    auto at_least = [](int a, int b) { return a > b ? a : b; };
+    L.patch_rows = rows;
+    const int patches = kMbWaves * rows * 32 * 4;
+    if (last) {   // kr and y; once both are dead the matrix, and after it g's tile, then q's
+      const int rows_gq = M * (d > dv ? d : dv) * 2;
+      L.k = take(at_least(M * (d + dv) * 2, mat + rows_gq));
+      L.y = L.k + M * d * 2;
+      L.mat0 = L.mat1 = L.k;
+      L.q = L.g = L.k + mat;
+      L.patch = take(patches);
+    } else {
+      L.k = take(M * d * 2);
+      L.g = take(M * d * 2);
+      L.q = take(at_least(M * d * 2 + patches, mat));
+      L.patch = L.q + M * d * 2;
+      L.mat0 = L.mat1 = L.q;
+      L.lse = take(M * 4);
+      L.part = take(4 * M * 4);
+    }
+    L.e = take(M * 4);
+    L.rs = take(M * 4);
+    L.total = off;
+    if (best.total == 0 || 160 * 1024 / L.total > 160 * 1024 / best.total) best = L;
+  }
+  return best;
 }
 
 // Stage the m rows of W 16-bit values (row r: src + r rs) into a tile whose chunk c of row r sits at chunk
@@ -436,23 +480,65 @@ __global__ __launch_bounds__(64 * kMbWaves, TWO && !LAST ? 4 : 2) void lstep_mb_
 }
 
 
+// Sums of an accumulator block's 16 rows over the 32 lanes of each half: lane l gets the total of one row (lanes l and
+// l ^ 1 the same), 32-row index mb_lane_sums_row(l).  One permlane16 swap halves the registers, then every step
+// keeps half of them, by a lane bit, and adds the mirrored lane's other half: 38 vector instructions.
+__device__ __forceinline__ int mb_lane_sums_row(int lane) {
+  const int r = ((lane & 8) >> 1) + ((lane & 4) >> 1) + ((lane & 2) >> 1) + ((lane & 16) >> 1);   // accumulator row
+  return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+}
+__device__ __forceinline__ float mb_lane_sums(const f32x16& t, int lane) {
+  float s[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {   // even 16-lane rows: accumulator row r, odd ones: r + 8
+    const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(t[r]), __float_as_uint(t[r + 8]), false, false);
+    s[r] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+  }
+  auto step = [&](int n, int bit, auto ctrl) __attribute__((always_inline)) {
+    const bool up = (lane & bit) != 0;
+#pragma unroll
+    for (int r = 0; r < n; ++r) {
+      const float keep = up ? s[r + n] : s[r], give = up ? s[r] : s[r + n];
+      s[r] = keep + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(give), decltype(ctrl)::value, 0xf, 0xf, true));
+    }
+  };
+  step(4, 8, std::integral_constant<int, 0x140>{});   // row_mirror: lane 15 - j
+  step(2, 4, std::integral_constant<int, 0x141>{});   // row_half_mirror: 7 - j
+  step(1, 2, std::integral_constant<int, 0x1b>{});    // quad_perm: 3 - j
+  return s[0] + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(s[0]), 0xb1, 0xf, 0xf, true));   // j ^ 1
+}
+
 // Backward of the multi-block L-step (the gradient autograd takes through vmonarch.py:51-63 with the entropy
 // bias detached, vmonarch.py:26), one 4-wave workgroup per grid column as the forward, with g the upstream
 // gradient rows (dz rows i when last, du rows k otherwise) staged beside q, kr (and y):
 //   last:  da[i,k] = g_i . y_k,  rs_i = sum_k a da,  dl = scale a (da - rs_i)
-//          pass A (wave = query block, one query row per lane): S^T and DA^T blocks -> lse_i, rs_i, then
-//          dq^T += Kr^T dl^T;  pass B (wave = key block, one key per lane): L and DA blocks ->
-//          dy^T += G^T a, dkr^T += Q^T dl
+//          query blocks (one query row per lane): S^T and DA^T blocks -> lse_i, rs_i, dl, dq^T += Kr^T dl^T;
+//          key blocks: dy^T += G^T a, dkr^T += Q^T dl
 //   else:  c_k = sum_i a, gv_k = sum_i a (g_k . q_i), f_k = scale / max(c_k, mcm),
 //          dc_k = -[c_k >= mcm] gv_k f_k / max(c_k, mcm),  da[i,k] = f_k (g_k . q_i) + dc_k
-//          pass 0 (query blocks): lse_i;  pass 1 (key blocks): c_k, gv_k -> f_k, dc_k;
-//          pass 2 (query blocks): rs_i, dq^T += Kr^T dl^T + G^T (a f)^T;  pass 3 (key blocks): dkr^T += Q^T dl
-// Every m x m block is recomputed where an orientation needs it (the MFMAs are cheap next to the column's
-// HBM traffic); the attention is exp2(logit - lse_i), exactly normalised.  MFMA operands a, dl and a f are
+//          query blocks: lse_i;  key blocks (one key per lane): a, g_k . q_i -> c_k, gv_k, f_k, dc_k, da, each
+//          wave's part of rs_i, then dl, dkr^T += Q^T dl;  query blocks: dq^T += Kr^T dl^T + G^T (a f)^T
+// One block per wave: the a and da blocks are formed once, in one orientation, and reach the other as rounded MFMA
+// operands through LDS matrices (mb_layout_bwd1).  Recomputing them in the second orientation, as this kernel did
+// before, took 80 / 88 (last / otherwise) MFMAs and as many operand reads per block pair at 128-wide heads instead of
+// 40 / 48.  What bounds a column is its chain (loads, passes, stores), so what counts most is a second column per CU
+// to overlap it with (73-80 KB of LDS and 256 registers up to 96 frames; the last step up to 128) and no HBM round
+// trips inside it (the rows dq is added to are read ahead).  12 heads x ~32760 tokens, 128-wide, non-last / last, us:
+// 65 frames 526 / 347 -> 232 / 235, 96 frames 381 / 269 -> 185 / 188 (4.4 TB/s of the algorithmic bytes), 128 frames
+// 344 / 251 -> 248 / 187.  The two-block kernels (TWO) recompute: their operands change hands through the row-store
+// patches; reading dq's rows ahead took their non-last step from 318 to 289 us at 33 frames, 194 to 172 at 64.  The attention is exp2(logit - lse_i),
+// exactly normalised.  MFMA operands a, dl and a f are
 // rounded to the 16-bit type, the sums rs, c, gv kept in fp32 from the fp32 attention.  dq (fp32) is added
 // to or overwritten, d out (the 16-bit type) written; rows past m carry zero attention and are not stored.
-template <bool F16, int D, int DV, bool LAST, bool TWO, bool CT>
-__global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams p) {
+// MBX: the most row blocks it takes (2 with TWO).
+template <int D, int DV, bool LAST, bool TWO, int MBX>
+constexpr int mb_bwd_min_waves() {
+  if (TWO) return 2;
+  if (D <= 32 && (!LAST || DV <= 32)) return MBX == 2 ? 4 : MBX == 3 ? 3 : 2;   // narrow tiles: many columns per CU
+  return LAST || MBX < 4 || D < 128 ? 2 : 1;
+}
+template <bool F16, int D, int DV, bool LAST, bool TWO, bool CT, int MBX>
+__global__ __launch_bounds__(64 * kMbWaves, (mb_bwd_min_waves<D, DV, LAST, TWO, MBX>())) void lstep_mb_bwd_kernel(LBParams p) {
   using E = Elem<F16>;
   using T = typename E::T;
   using V8 = typename E::V8;
@@ -467,7 +553,7 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
   VMO_LDS char* sm = (VMO_LDS char*)smem_raw;
 
   const int m = p.m, MB = (m + 31) / 32, M = 32 * MB;
-  const MbLayout Lo = mb_layout(m, DK, DVK, LAST, true, CT);
+  const MbLayout Lo = TWO ? mb_layout(m, DK, DVK, LAST, true, CT) : mb_layout_bwd1(m, DK, DVK, LAST);
   VMO_LDS char* q_t = sm + Lo.q;
   VMO_LDS char* k_t = sm + Lo.k;
   VMO_LDS char* y_t = sm + Lo.y;
@@ -479,8 +565,7 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
   VMO_LDS float* dc_t = (VMO_LDS float*)(sm + Lo.dc);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int hl = lane >> 5, l32 = lane & 31;
-  const bool half_patch = mb_bwd_patch_rows(LAST, M) == 16;
-  VMO_LDS float* patch = (VMO_LDS float*)(sm + Lo.patch + wave * mb_bwd_patch_rows(LAST, M) * 32 * 4);
+  VMO_LDS float* patch = (VMO_LDS float*)(sm + Lo.patch + wave * Lo.patch_rows * 32 * 4);
 
   const int col = blockIdx.x, bh = col / p.bs, j = col % p.bs, hh = bh % p.heads, bb = bh / p.heads;
   const int64_t q_rs = (int64_t)p.bs * p.q_sn, o_rs = (int64_t)p.bs * p.out_sn, g_rs = (int64_t)p.bs * p.g_sn;
@@ -491,15 +576,32 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
   float* dqcol = p.dq + bb * p.dq_sb + hh * p.dq_sh + (int64_t)j * p.dq_sn;
   T* dcol = (T*)p.dout + bb * p.do_sb + hh * p.do_sh + (int64_t)j * p.do_sn;
 
-  mb_stage<T, DK, D, CT>(qcol, q_rs, m, q_t, wave, lane);
+  constexpr bool ROWS_IN_REGS = LAST && !TWO;   // the wave's q and g rows as MFMA operands, read from HBM
+  V8 q_rows[ROWS_IN_REGS ? NDS : 1], g_rows[ROWS_IN_REGS ? NDSV : 1];
+  if constexpr (ROWS_IN_REGS) {
+    const int r = 32 * wave + l32, rr = r < m ? r : m - 1;
+    const bool g_ok = r < m && (int64_t)r * p.bs + j >= p.skip;   // (z rows of tokens < skip are the recompute's)
+#pragma unroll
+    for (int ds = 0; ds < NDS; ++ds) {
+      const V8 v = *(const V8*)(qcol + rr * q_rs + 16 * ds + 8 * hl);
+      q_rows[ds] = r < m ? v : V8{};
+    }
+#pragma unroll
+    for (int ds = 0; ds < NDSV; ++ds) {
+      const V8 v = *(const V8*)(gcol + rr * g_rs + 16 * ds + 8 * hl);
+      g_rows[ds] = g_ok ? v : V8{};
+    }
+  } else {
+    mb_stage<T, DK, D, CT>(qcol, q_rs, m, q_t, wave, lane);
+    mb_stage<T, GWK, GW, CT>(gcol, g_rs, m, g_t, wave, lane);
+  }
   mb_stage<T, DK, D, CT>(ocol, o_rs, m, k_t, wave, lane);
   if constexpr (LAST) mb_stage<T, DVK, DV, CT>(ocol + D, o_rs, m, y_t, wave, lane);
-  mb_stage<T, GWK, GW, CT>(gcol, g_rs, m, g_t, wave, lane);
   const float* ep = p.ent + bb * p.ent_sb + hh * p.ent_sh + j;
   for (int k = tid; k < M; k += 64 * kMbWaves) e_t[k] = k < m ? ep[(int64_t)k * p.bs] * kLog2e : -1.0e30f;
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if constexpr (LAST) {   // z rows of tokens < skip are the recompute's: no gradient reaches the L-path
+  if constexpr (LAST && TWO) {   // z rows of tokens < skip are the recompute's: no gradient reaches the L-path
     constexpr int CH = RBG / 16;
     for (int idx = tid; idx < m * CH; idx += 64 * kMbWaves) {
       const int r = idx / CH;
@@ -542,10 +644,10 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
     return x;
   };
   // query block's row LSE from its S^T blocks (kept in x for the caller)
-  auto row_lse = [&](const V8 (&qb)[NDS], f32x16 (&x)[kMbMaxBlocks]) __attribute__((always_inline)) {
+  auto row_lse = [&](const V8 (&qb)[NDS], f32x16 (&x)[MBX]) __attribute__((always_inline)) {
     float mx = -3.0e38f;
 #pragma unroll
-    for (int kb = 0; kb < kMbMaxBlocks; ++kb) {
+    for (int kb = 0; kb < MBX; ++kb) {
       if (kb >= MB) break;
       x[kb] = s_block(kb, qb);
 #pragma unroll
@@ -554,7 +656,7 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
     mx = wave_max32(mx);
     float sum = 0.f;
 #pragma unroll
-    for (int kb = 0; kb < kMbMaxBlocks; ++kb) {
+    for (int kb = 0; kb < MBX; ++kb) {
       if (kb >= MB) break;
 #pragma unroll
       for (int r = 0; r < 16; ++r) sum += fast_exp2(x[kb][r] - mx);
@@ -567,12 +669,48 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
   };
   const bool row_ok = 32 * blk + l32 < m;   // this lane's query row (query-block passes) or key (key-block passes)
   const int nrows = busy ? min(32, m - 32 * blk) : 0;
-  // row stores through the patch: whole (32 rows) or half (16 rows at a time)
+  // row stores through the patch: whole (32 rows), or 16 or 8 rows at a time
   auto store_rows = [&](auto cw_tag, const f32x16* acc, int nacc, int mode, char* row0, int64_t stride, int nr)
       __attribute__((always_inline)) {
     constexpr int CWS = decltype(cw_tag)::value;
-    if (half_patch) store_acc_rows<F16, CWS, 16>(patch, acc, nacc, 1.f, mode, row0, stride, nr, lane);
-    else store_acc_rows<F16, CWS, 32>(patch, acc, nacc, 1.f, mode, row0, stride, nr, lane);
+    if (Lo.patch_rows == 32) store_acc_rows<F16, CWS, 32>(patch, acc, nacc, 1.f, mode, row0, stride, nr, lane);
+    else if (TWO || Lo.patch_rows == 16) store_acc_rows<F16, CWS, 16>(patch, acc, nacc, 1.f, mode, row0, stride, nr, lane);
+    else store_acc_rows<F16, CWS, 8>(patch, acc, nacc, 1.f, mode, row0, stride, nr, lane);
+  };
+  // The rows an fp32 result is added to, read ahead of the products that form it instead of one HBM round trip per
+  // 32-column block at the end (base[a][i]: row lane / 8 + 8 i, columns CWD a + 4 (lane % 8) ..), and the store of
+  // acc plus them.
+  auto load_base = [&](auto& base, auto n_tag, const char* row0, int64_t stride, int nr) __attribute__((always_inline)) {
+    constexpr int N = decltype(n_tag)::value;
+#pragma unroll
+    for (int a = 0; a < N; ++a)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int rr = (lane >> 3) + 8 * i, cc = lane & 7;
+        base[a][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (rr < nr && 4 * cc < CWD) base[a][i] = *(const f32x4*)(row0 + rr * stride + (int64_t)(CWD * a + 4 * cc) * 4);
+      }
+  };
+  auto store_rows_added = [&](const auto& acc, const auto& base, auto n_tag, char* row0, int64_t stride, int nr)
+      __attribute__((always_inline)) {
+    constexpr int N = decltype(n_tag)::value;
+    const int pr_max = Lo.patch_rows, cc = lane & 7;
+#pragma unroll
+    for (int a = 0; a < N; ++a)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {   // 8 rows through the patch at a time: rows 8 i .. 8 i + 7
+        if ((l32 >> 3) == i) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *(VMO_LDS f32x4*)(patch + ((8 * i + (l32 & 7)) % pr_max) * 32 + ((2 * g + hl) ^ (l32 & 7)) * 4) =
+                f32x4{acc[a][4 * g], acc[a][4 * g + 1], acc[a][4 * g + 2], acc[a][4 * g + 3]};
+        }
+        asm volatile("" ::: "memory");   // (lanes read what other lanes wrote, as in store_acc_rows)
+        const int rr = (lane >> 3) + 8 * i;
+        const f32x4 v = *(const VMO_LDS f32x4*)(patch + (rr % pr_max) * 32 + (cc ^ (rr & 7)) * 4);
+        if (rr < nr && 4 * cc < CWD) *(f32x4*)(row0 + rr * stride + (int64_t)(CWD * a + 4 * cc) * 4) = base[a][i] + v;
+        asm volatile("" ::: "memory");
+      }
   };
   // The two-block kernels (TWO) give each wave a (query block ib, key block kb) pair.  pair_lse: the row LSE of
   // the query rows from the S^T blocks of the pairs (each wave's x), as the partial max and sum of each key
@@ -604,6 +742,44 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
     if (hl == 0) part[kb * M + 32 * ib + l32] = v;
     __syncthreads();
     return part[32 * ib + l32] + part[M + 32 * ib + l32];
+  };
+
+  // One-block-per-wave passes.  put_mat: this wave's block row (lane: row l32 of block blk, accumulator order over
+  // the columns) of a 16-bit matrix into LDS rows of kMbMatRow bytes, chunks swizzled like a tile's.  mat_product:
+  // acc[f][c] (+)= sum_r tile[r][f] mat[r][c] for the columns c of block blk: both operands by transposed reads, in
+  // the same row order.
+  auto put_mat = [&](VMO_LDS char* mat, const V8 (&B)[MBX][2]) __attribute__((always_inline)) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    VMO_LDS char* row = mat + (32 * blk + l32) * kMbMatRow + hl * 8;
+    const int sw = swz_rows<kMbMatRow>(l32);
+#pragma unroll
+    for (int cb = 0; cb < MBX; ++cb) {
+      if (cb >= MB) break;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {   // columns 32 cb + 8 g + 4 hl .. + 3: chunk 4 cb + g, half hl
+        const u32x4 w = __builtin_bit_cast(u32x4, B[cb][g >> 1]);
+        *(VMO_LDS u32x2*)(row + ((4 * cb + g) ^ sw) * 16) = u32x2{w[2 * (g & 1)], w[2 * (g & 1) + 1]};
+      }
+    }
+  };
+  auto mat_product = [&](auto& acc, auto n_tag, auto rb_tag, const VMO_LDS char* tile, const VMO_LDS char* mat, bool zero)
+      __attribute__((always_inline)) {
+    constexpr int N = decltype(n_tag)::value, RB = decltype(rb_tag)::value;
+    if (zero) {
+#pragma unroll
+      for (int a = 0; a < N; ++a) acc[a] = f32x16{};
+    }
+#pragma unroll
+    for (int rb = 0; rb < MBX; ++rb) {
+      if (rb >= MB) break;
+#pragma unroll
+      for (int h2 = 0; h2 < 2; ++h2) {
+        const V8 b = mb_tr8<V8, kMbMatRow, false>(mat, rb, m, lane, blk, h2);
+#pragma unroll
+        for (int a = 0; a < N; ++a) acc[a] = E::mfma(mb_tr8<V8, RB, false>(tile, rb, m, lane, a, h2), b, acc[a]);
+      }
+    }
   };
 
   if constexpr (LAST) {
@@ -711,103 +887,80 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
         store_rows(std::integral_constant<int, CWD>{}, acck, NH, kGradStore, (char*)(dcol + 32 * kq * do_rs + 32 * iq * NH),
                    do_rs * 2, nr);
       }
-      return;
-    }
-    // ---- pass A: one query row per lane
-    if (busy) {
-      V8 qb[NDS];
-      load_rows(qb, q_t, blk);
-      f32x16 x[kMbMaxBlocks];
-      const float lse = row_lse(qb, x);
-      auto da_block = [&](int kb) __attribute__((always_inline)) {   // DA^T[k][i] = y_k . g_i (g rows read at each use)
-        f32x16 d = f32x16{};
+    } else {
+      // ---- one query row per lane: a and da against every key block, rs_i, dl, dq; the other orientation's products
+      // then take a and dl from an LDS matrix [i][k] each
+      V8 P[MBX][2], A[MBX][2];
+      if (busy) {
+        f32x16 x[MBX], d[MBX];
+        const float lse = row_lse(q_rows, x);
+        float rs = 0.f;
 #pragma unroll
-        for (int ds = 0; ds < NDSV; ++ds)
-          d = E::mfma(mb_row8<V8, RBY, CT>(y_t, kb, m, l32, hl, ds), mb_row8<V8, RBY, CT>(g_t, blk, m, l32, hl, ds),
-                      d);
-        return d;
+        for (int kb = 0; kb < MBX; ++kb) {
+          if (kb >= MB) break;
+          d[kb] = f32x16{};   // DA^T[k][i] = y_k . g_i
+#pragma unroll
+          for (int ds = 0; ds < NDSV; ++ds) d[kb] = E::mfma(mb_row8<V8, RBY, CT>(y_t, kb, m, l32, hl, ds), g_rows[ds], d[kb]);
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            x[kb][r] = row_ok ? fast_exp2(x[kb][r] - lse) : 0.f;   // (rows past m: no attention)
+            rs = fmaf(x[kb][r], d[kb][r], rs);
+          }
+        }
+        rs = wave_sum32(rs);
+        f32x16 accq[ND];
+#pragma unroll
+        for (int a = 0; a < ND; ++a) accq[a] = f32x16{};
+#pragma unroll
+        for (int kb = 0; kb < MBX; ++kb) {
+          if (kb >= MB) break;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) d[kb][r] = p.scale * x[kb][r] * (d[kb][r] - rs);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            P[kb][h] = mb_pack<T, V8>(d[kb], h, 1.f);
+            A[kb][h] = mb_pack<T, V8>(x[kb], h, 1.f);
+          }
+#pragma unroll
+          for (int a = 0; a < ND; ++a) {
+            accq[a] = E::mfma(mb_tr8<V8, RBD, CT>(k_t, kb, m, lane, a, 0), P[kb][0], accq[a]);
+            accq[a] = E::mfma(mb_tr8<V8, RBD, CT>(k_t, kb, m, lane, a, 1), P[kb][1], accq[a]);
+          }
+        }
+        store_rows(std::integral_constant<int, CWD>{}, accq, ND, dq_mode, (char*)(dqcol + 32 * blk * dq_rs), dq_rs * 4, nrows);
+      }
+      // this wave's rows (operands over W columns) into a tile of W-wide rows
+      auto put_rows = [&](VMO_LDS char* tile, auto rb_tag, const auto& rows, int n) __attribute__((always_inline)) {
+        constexpr int RB = decltype(rb_tag)::value;
+        VMO_LDS char* row = tile + (32 * blk + l32) * RB;
+#pragma unroll
+        for (int ds = 0; ds < RB / 32; ++ds)   // (a 16-wide tensor in a 32-wide tile: its chunks twice)
+          *(VMO_LDS V8*)(row + ((2 * ds + hl) ^ swz_rows<RB>(l32)) * 16) = rows[ds % n];
       };
-      float rs = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < kMbMaxBlocks; ++kb) {
-        if (kb >= MB) break;
-        const f32x16 d = da_block(kb);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) rs = fmaf(fast_exp2(x[kb][r] - lse), d[r], rs);
+      __syncthreads();   // every wave is done with kr and y
+      if (busy) {
+        put_mat(sm + Lo.mat0, A);
+        put_rows(g_t, std::integral_constant<int, RBG>{}, g_rows, NDSV);
       }
-      rs = wave_sum32(rs);
-      if (hl == 0) {
-        lse_t[32 * blk + l32] = row_ok ? lse : 1.0e30f;
-        rs_t[32 * blk + l32] = row_ok ? rs : 0.f;
+      __syncthreads();
+      if (busy) {   // dy^T[dv][k] += sum_i g^T[dv][i] a[i][k]
+        f32x16 accy[NV];
+        mat_product(accy, std::integral_constant<int, NV>{}, std::integral_constant<int, RBG>{}, g_t, sm + Lo.mat0, true);
+        store_rows(std::integral_constant<int, CWV>{}, accy, NV, kGradStore, (char*)(dcol + 32 * blk * do_rs + D),
+                   do_rs * 2, nrows);
       }
-      f32x16 accq[ND];
-#pragma unroll
-      for (int a = 0; a < ND; ++a) accq[a] = f32x16{};
-#pragma unroll
-      for (int kb = 0; kb < kMbMaxBlocks; ++kb) {
-        if (kb >= MB) break;
-        f32x16 dl = da_block(kb);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) dl[r] = p.scale * fast_exp2(x[kb][r] - lse) * (dl[r] - rs);
-        const V8 P0 = mb_pack<T, V8>(dl, 0, 1.f), P1 = mb_pack<T, V8>(dl, 1, 1.f);
-#pragma unroll
-        for (int a = 0; a < ND; ++a) {
-          accq[a] = E::mfma(mb_tr8<V8, RBD, CT>(k_t, kb, m, lane, a, 0), P0, accq[a]);
-          accq[a] = E::mfma(mb_tr8<V8, RBD, CT>(k_t, kb, m, lane, a, 1), P1, accq[a]);
-        }
+      __syncthreads();
+      if (busy) {
+        put_mat(sm + Lo.mat1, P);
+        put_rows(q_t, std::integral_constant<int, RBD>{}, q_rows, NDS);
       }
-      store_rows(std::integral_constant<int, CWD>{}, accq, ND, dq_mode, (char*)(dqcol + 32 * blk * dq_rs), dq_rs * 4, nrows);
-    }
-    __syncthreads();
-    // ---- pass B: one key per lane, as two sweeps over the query blocks (dy, then dkr: holding both accumulator
-    // sets at once spills at 128 / 128, and recomputing the attention block is cheap next to the HBM traffic)
-    if (busy) {
-      const float ek = e_t[32 * blk + l32];
-      f32x16 accy[NV];
-#pragma unroll
-      for (int a = 0; a < NV; ++a) accy[a] = f32x16{};
-#pragma unroll
-      for (int ib = 0; ib < kMbMaxBlocks; ++ib) {
-        if (ib >= MB) break;
-        const f32x16 at = attn_block(ib, blk, ek);
-        // dy^T[dv][k] += sum_i g^T[dv][i] a[i][k]
-        const V8 A0 = mb_pack<T, V8>(at, 0, 1.f), A1 = mb_pack<T, V8>(at, 1, 1.f);
-#pragma unroll
-        for (int a = 0; a < NV; ++a) {
-          accy[a] = E::mfma(mb_tr8<V8, RBY, CT>(g_t, ib, m, lane, a, 0), A0, accy[a]);
-          accy[a] = E::mfma(mb_tr8<V8, RBY, CT>(g_t, ib, m, lane, a, 1), A1, accy[a]);
-        }
+      __syncthreads();
+      if (busy) {   // dkr^T[d][k] += sum_i q^T[d][i] dl[i][k]
+        f32x16 acck[ND];
+        mat_product(acck, std::integral_constant<int, ND>{}, std::integral_constant<int, RBD>{}, q_t, sm + Lo.mat1, true);
+        store_rows(std::integral_constant<int, CWD>{}, acck, ND, kGradStore, (char*)(dcol + 32 * blk * do_rs), do_rs * 2,
+                   nrows);
       }
-      store_rows(std::integral_constant<int, CWV>{}, accy, NV, kGradStore, (char*)(dcol + 32 * blk * do_rs + D),
-                 do_rs * 2, nrows);
-      f32x16 acck[ND];
-#pragma unroll
-      for (int a = 0; a < ND; ++a) acck[a] = f32x16{};
-#pragma unroll
-      for (int ib = 0; ib < kMbMaxBlocks; ++ib) {
-        if (ib >= MB) break;
-        const f32x16 at = attn_block(ib, blk, ek);
-        // DA[i][k] = g_i . y_k, dl = scale a (da - rs_i)
-        f32x16 dl = f32x16{};
-#pragma unroll
-        for (int ds = 0; ds < NDSV; ++ds)
-          dl = E::mfma(mb_row8<V8, RBY, CT>(g_t, ib, m, l32, hl, ds), mb_row8<V8, RBY, CT>(y_t, blk, m, l32, hl, ds),
-                       dl);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4 rv = *(const VMO_LDS f32x4*)(rs_t + 32 * ib + 8 * g + 4 * hl);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) dl[4 * g + e] = p.scale * at[4 * g + e] * (dl[4 * g + e] - rv[e]);
-        }
-        const V8 P0 = mb_pack<T, V8>(dl, 0, 1.f), P1 = mb_pack<T, V8>(dl, 1, 1.f);
-#pragma unroll
-        for (int a = 0; a < ND; ++a) {
-          acck[a] = E::mfma(mb_tr8<V8, RBD, CT>(q_t, ib, m, lane, a, 0), P0, acck[a]);
-          acck[a] = E::mfma(mb_tr8<V8, RBD, CT>(q_t, ib, m, lane, a, 1), P1, acck[a]);
-        }
-      }
-      store_rows(std::integral_constant<int, CWD>{}, acck, ND, kGradStore, (char*)(dcol + 32 * blk * do_rs), do_rs * 2,
-                 nrows);
     }
   } else {
     if constexpr (TWO) {
@@ -857,6 +1010,10 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
       __syncthreads();
       // ---- pass 2: rs_i from the two key blocks' partials, then dq (query block ib, column half kb)
       {
+        char* const dq0 = (char*)(dqcol + 32 * ib * dq_rs + 32 * kb * NH);
+        const int dq_nr = min(32, m - 32 * ib);
+        f32x4 base[NH][4];
+        if (dq_mode == kGradAddF32) load_base(base, std::integral_constant<int, NH>{}, dq0, dq_rs * 4, dq_nr);
         f32x16 x = s_block(kb, qb);
         const float lse = lse_t[32 * ib + l32];
 #pragma unroll
@@ -909,8 +1066,8 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
           }
         }
         __syncthreads();   // every wave is done with xch: the patches may reuse it
-        store_rows(std::integral_constant<int, CWD>{}, accq, NH, dq_mode, (char*)(dqcol + 32 * ib * dq_rs + 32 * kb * NH),
-                   dq_rs * 4, min(32, m - 32 * ib));
+        if (dq_mode == kGradAddF32) store_rows_added(accq, base, std::integral_constant<int, NH>{}, dq0, dq_rs * 4, dq_nr);
+        else store_rows(std::integral_constant<int, CWD>{}, accq, NH, dq_mode, dq0, dq_rs * 4, dq_nr);
       }
       __syncthreads();   // the patches are free again for xch, and rs_t is complete
       // ---- pass 3: dkr (key block kq, column half iq) over the two query blocks
@@ -955,143 +1112,119 @@ __global__ __launch_bounds__(64 * kMbWaves, 2) void lstep_mb_bwd_kernel(LBParams
       }
       return;
     }
-    // ---- pass 0: row LSE (query blocks)
+    // ---- row LSE (query blocks)
     if (busy) {
       V8 qb[NDS];
       load_rows(qb, q_t, blk);
-      f32x16 x[kMbMaxBlocks];
+      f32x16 x[MBX];
       const float lse = row_lse(qb, x);
       if (hl == 0) lse_t[32 * blk + l32] = row_ok ? lse : 1.0e30f;
     }
     __syncthreads();
-    // ---- pass 1: column mass c_k and gv_k = sum_i a (g_k . q_i) (key blocks) -> f_k, dc_k
+    // ---- one key per lane: a and g_k . q_i against every query block, column mass c_k and gv_k = sum_i a (g_k . q_i)
+    // -> f_k, dc_k (all in the key's lanes); then rs_i, a sum over the keys, from each wave's partial per query row
+    V8 P[MBX][2], F[MBX][2];
+    f32x16 at[MBX], da[MBX];
+    VMO_LDS float* const wpart = part + blk * M;   // this wave's sums over its 32 keys, per query row
     if (busy) {
-      V8 gop[NDS];
+      V8 kop[NDS], gop[NDS];
+      load_rows(kop, k_t, blk);
       load_rows(gop, g_t, blk);
       const float ek = e_t[32 * blk + l32];
       float cs = 0.f, gv = 0.f;
 #pragma unroll
-      for (int ib = 0; ib < kMbMaxBlocks; ++ib) {
+      for (int ib = 0; ib < MBX; ++ib) {
         if (ib >= MB) break;
-        const f32x16 at = attn_block(ib, blk, ek);
-        f32x16 gq = f32x16{};   // GQ[i][k] = q_i . g_k
+        at[ib] = f32x16{};
+        da[ib] = f32x16{};   // GQ[i][k] = q_i . g_k
 #pragma unroll
-        for (int ds = 0; ds < NDS; ++ds) gq = E::mfma(mb_row8<V8, RBD, CT>(q_t, ib, m, l32, hl, ds), gop[ds], gq);
+        for (int ds = 0; ds < NDS; ++ds) {
+          const V8 qr = mb_row8<V8, RBD, CT>(q_t, ib, m, l32, hl, ds);
+          at[ib] = E::mfma(qr, kop[ds], at[ib]);
+          da[ib] = E::mfma(qr, gop[ds], da[ib]);
+        }
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          cs += at[r];
-          gv = fmaf(at[r], gq[r], gv);
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 lv = *(const VMO_LDS f32x4*)(lse_t + 32 * ib + 8 * g + 4 * hl);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int r = 4 * g + e;
+            at[ib][r] = fast_exp2(fmaf(at[ib][r], c, ek - lv[e]));
+            cs += at[ib][r];
+            gv = fmaf(at[ib][r], da[ib][r], gv);
+          }
         }
       }
       cs = wave_sum32(cs);
       gv = wave_sum32(gv);
-      const float cm = fmaxf(cs, p.min_col_mass), f = p.scale / cm;
-      if (hl == 0) {
-        f_t[32 * blk + l32] = f;
-        dc_t[32 * blk + l32] = (row_ok && cs >= p.min_col_mass) ? -gv * f / cm : 0.f;
+      const float cm = fmaxf(cs, p.min_col_mass), fk = row_ok ? p.scale / cm : 0.f;
+      const float dck = row_ok && cs >= p.min_col_mass ? -gv * fk / cm : 0.f;
+#pragma unroll
+      for (int ib = 0; ib < MBX; ++ib) {
+        if (ib >= MB) break;
+        f32x16 t;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          da[ib][r] = fmaf(fk, da[ib][r], dck);
+          t[r] = at[ib][r] * da[ib][r];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) F[ib][h] = mb_pack<T, V8>(at[ib], h, fk);
+        const float sum = mb_lane_sums(t, lane);   // over the wave's keys (lanes)
+        if ((lane & 1) == 0) wpart[32 * ib + mb_lane_sums_row(lane)] = sum;
       }
     }
     __syncthreads();
-    // ---- pass 2: rs_i and dq (query blocks)
-    if (busy) {
-      V8 qb[NDS];
-      load_rows(qb, q_t, blk);
-      f32x16 x[kMbMaxBlocks];
-      const float lse = lse_t[32 * blk + l32];
-#pragma unroll
-      for (int kb = 0; kb < kMbMaxBlocks; ++kb) {
-        if (kb >= MB) break;
-        x[kb] = s_block(kb, qb);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[kb][r] = fast_exp2(x[kb][r] - lse);   // attn^T[k][i]
-      }
-      // da^T[k][i] = f_k (g_k . q_i) + dc_k
-      auto da_block = [&](int kb) __attribute__((always_inline)) {
-        f32x16 d = f32x16{};
-#pragma unroll
-        for (int ds = 0; ds < NDS; ++ds) d = E::mfma(mb_row8<V8, RBD, CT>(g_t, kb, m, l32, hl, ds), qb[ds], d);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4 fv = *(const VMO_LDS f32x4*)(f_t + 32 * kb + 8 * g + 4 * hl);
-          const f32x4 cv = *(const VMO_LDS f32x4*)(dc_t + 32 * kb + 8 * g + 4 * hl);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) d[4 * g + e] = fmaf(fv[e], d[4 * g + e], cv[e]);
-        }
-        return d;
-      };
+    if (tid < M) {
       float rs = 0.f;
-#pragma unroll
-      for (int kb = 0; kb < kMbMaxBlocks; ++kb) {
-        if (kb >= MB) break;
-        const f32x16 d = da_block(kb);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) rs = fmaf(x[kb][r], d[r], rs);
-      }
-      rs = wave_sum32(rs);
-      if (hl == 0) rs_t[32 * blk + l32] = row_ok ? rs : 0.f;
-      f32x16 accq[ND];
-#pragma unroll
-      for (int a = 0; a < ND; ++a) accq[a] = f32x16{};
-#pragma unroll
-      for (int kb = 0; kb < kMbMaxBlocks; ++kb) {
-        if (kb >= MB) break;
-        f32x16 dl = da_block(kb), af;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4 fv = *(const VMO_LDS f32x4*)(f_t + 32 * kb + 8 * g + 4 * hl);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int r = 4 * g + e;
-            af[r] = x[kb][r] * fv[e];
-            dl[r] = p.scale * x[kb][r] * (dl[r] - rs);
-          }
-        }
-        const V8 P0 = mb_pack<T, V8>(dl, 0, 1.f), P1 = mb_pack<T, V8>(dl, 1, 1.f);
-        const V8 F0 = mb_pack<T, V8>(af, 0, 1.f), F1 = mb_pack<T, V8>(af, 1, 1.f);
-#pragma unroll
-        for (int a = 0; a < ND; ++a) {
-          accq[a] = E::mfma(mb_tr8<V8, RBD, CT>(k_t, kb, m, lane, a, 0), P0, accq[a]);
-          accq[a] = E::mfma(mb_tr8<V8, RBD, CT>(k_t, kb, m, lane, a, 1), P1, accq[a]);
-          accq[a] = E::mfma(mb_tr8<V8, RBD, CT>(g_t, kb, m, lane, a, 0), F0, accq[a]);
-          accq[a] = E::mfma(mb_tr8<V8, RBD, CT>(g_t, kb, m, lane, a, 1), F1, accq[a]);
-        }
-      }
-      store_acc_rows<F16, CWD>(patch, accq, ND, 1.f, dq_mode, (char*)(dqcol + 32 * blk * dq_rs), dq_rs * 4, nrows, lane);
+      for (int w = 0; w < MB; ++w) rs += part[w * M + tid];
+      rs_t[tid] = tid < m ? rs : 0.f;
     }
     __syncthreads();
-    // ---- pass 3: dkr (key blocks)
-    if (busy) {
-      V8 gop[NDS];
-      load_rows(gop, g_t, blk);
-      const float ek = e_t[32 * blk + l32];
-      const float fk = f_t[32 * blk + l32], dck = dc_t[32 * blk + l32];
+    f32x4 base[ND][4];
+    const bool add_q = dq_mode == kGradAddF32;
+    if (busy) {   // dl; dkr^T[d][k] += sum_i q^T[d][i] dl[i][k]
       f32x16 acck[ND];
 #pragma unroll
       for (int a = 0; a < ND; ++a) acck[a] = f32x16{};
 #pragma unroll
-      for (int ib = 0; ib < kMbMaxBlocks; ++ib) {
+      for (int ib = 0; ib < MBX; ++ib) {
         if (ib >= MB) break;
-        const f32x16 at = attn_block(ib, blk, ek);
-        f32x16 dl = f32x16{};
-#pragma unroll
-        for (int ds = 0; ds < NDS; ++ds) dl = E::mfma(mb_row8<V8, RBD, CT>(q_t, ib, m, l32, hl, ds), gop[ds], dl);
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const f32x4 rv = *(const VMO_LDS f32x4*)(rs_t + 32 * ib + 8 * g + 4 * hl);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int r = 4 * g + e;
-            dl[r] = p.scale * at[r] * (fmaf(fk, dl[r], dck) - rv[e]);
+            da[ib][r] = p.scale * at[ib][r] * (da[ib][r] - rv[e]);
           }
         }
-        const V8 P0 = mb_pack<T, V8>(dl, 0, 1.f), P1 = mb_pack<T, V8>(dl, 1, 1.f);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) P[ib][h] = mb_pack<T, V8>(da[ib], h, 1.f);
 #pragma unroll
         for (int a = 0; a < ND; ++a) {
-          acck[a] = E::mfma(mb_tr8<V8, RBD, CT>(q_t, ib, m, lane, a, 0), P0, acck[a]);
-          acck[a] = E::mfma(mb_tr8<V8, RBD, CT>(q_t, ib, m, lane, a, 1), P1, acck[a]);
+          acck[a] = E::mfma(mb_tr8<V8, RBD, CT>(q_t, ib, m, lane, a, 0), P[ib][0], acck[a]);
+          acck[a] = E::mfma(mb_tr8<V8, RBD, CT>(q_t, ib, m, lane, a, 1), P[ib][1], acck[a]);
         }
       }
-      store_acc_rows<F16, CWD>(patch, acck, ND, 1.f, kGradStore, (char*)(dcol + 32 * blk * do_rs), do_rs * 2, nrows, lane);
+      if (add_q) load_base(base, std::integral_constant<int, ND>{}, (const char*)(dqcol + 32 * blk * dq_rs), dq_rs * 4, nrows);
+      store_rows(std::integral_constant<int, CWD>{}, acck, ND, kGradStore, (char*)(dcol + 32 * blk * do_rs), do_rs * 2, nrows);
+    }
+    __syncthreads();   // every wave is done with q and the patches
+    // ---- dq^T[d][i] += sum_k kr^T[d][k] dl[i][k] + g^T[d][k] (a f)[i][k], from an LDS matrix [k][i] each
+    if (busy) put_mat(sm + Lo.mat0, P);
+    __syncthreads();
+    f32x16 accq[ND];
+    if (busy) mat_product(accq, std::integral_constant<int, ND>{}, std::integral_constant<int, RBD>{}, k_t, sm + Lo.mat0, true);
+    __syncthreads();
+    if (busy) put_mat(sm + Lo.mat1, F);
+    __syncthreads();
+    if (busy) mat_product(accq, std::integral_constant<int, ND>{}, std::integral_constant<int, RBD>{}, g_t, sm + Lo.mat1, false);
+    __syncthreads();   // every wave is done with the matrix, which the patches overlay
+    if (busy) {
+      char* const row0 = (char*)(dqcol + 32 * blk * dq_rs);
+      if (add_q) store_rows_added(accq, base, std::integral_constant<int, ND>{}, row0, dq_rs * 4, nrows);
+      else store_rows(std::integral_constant<int, CWD>{}, accq, ND, dq_mode, row0, dq_rs * 4, nrows);
     }
   }
 }
@@ -1106,7 +1239,9 @@ static bool mb_dims(int d, int dv, bool last) {
 
 int mb_lstep_check(int m, int d, int dv, bool last, bool bwd) {
   if (!mb_dims(d, dv, last) || m < 1 || m > kMbMaxFrames) return 0;
-  return mb_layout(m, tile_w(d), last ? tile_w(dv) : 0, last, bwd, false).total <= 160 * 1024;
+  const int dk = tile_w(d), dvk = last ? tile_w(dv) : 0;
+  if (mb_layout(m, dk, dvk, last, bwd, false).total > 160 * 1024) return 0;
+  return !bwd || mb_layout_bwd1(m, dk, dvk, last).total <= 160 * 1024;
 }
 
 template <bool F16, int D, int DV, bool LAST, bool TWO, bool CT>
@@ -1161,10 +1296,11 @@ int mb_lstep_fwd(const LParams& p, bool f16, int d, int dv, bool last, hipStream
   return f16 ? dispatch_mb<true>(p, d, dv, last, s) : dispatch_mb<false>(p, d, dv, last, s);
 }
 
-template <bool F16, int D, int DV, bool LAST, bool TWO, bool CT>
+template <bool F16, int D, int DV, bool LAST, bool TWO, bool CT, int MBX>
 static int launch_mb_bwd_k(const LBParams& p, hipStream_t s) {
-  const int lds = mb_layout(p.m, tile_w(D), tile_w(DV), LAST, true, CT).total;
-  auto kern = lstep_mb_bwd_kernel<F16, D, DV, LAST, TWO, CT>;
+  const int lds = TWO ? mb_layout(p.m, tile_w(D), tile_w(DV), LAST, true, CT).total
+                      : mb_layout_bwd1(p.m, tile_w(D), tile_w(DV), LAST).total;
+  auto kern = lstep_mb_bwd_kernel<F16, D, DV, LAST, TWO, CT, MBX>;
   static std::atomic<int> lds_limit{65536};   // as in launch_mb, per kernel
   if (lds > lds_limit.load(std::memory_order_relaxed)) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
@@ -1176,19 +1312,22 @@ static int launch_mb_bwd_k(const LBParams& p, hipStream_t s) {
 }
 
 // Grids of two row blocks (33-64 frames) take the kernel whose passes split the block pairs over all four waves,
-// where the accumulator blocks split evenly (32-wide heads and 16-wide tiles have one block); larger grids keep
-// one block per wave.
+// where the accumulator blocks split evenly (32-wide heads and 16-wide tiles have one block); the others keep one
+// block per wave, up to three (96 frames: registers for two waves per SIMD at any head dim) or four.
 template <bool F16, int D, int DV, bool LAST>
 static int launch_mb_bwd(const LBParams& p, hipStream_t s) {
   constexpr bool TWO_OK = (tile_w(D) / 32) % 2 == 0 && (!LAST || (tile_w(DV) / 32) % 2 == 0);
   if constexpr (TWO_OK) {
     if ((p.m + 31) / 32 == 2) {
       if constexpr (mb_compact_built(D, DV, LAST))
-        if (p.m <= kMbCompactMaxFrames) return launch_mb_bwd_k<F16, D, DV, LAST, true, true>(p, s);
-      return launch_mb_bwd_k<F16, D, DV, LAST, true, false>(p, s);
+        if (p.m <= kMbCompactMaxFrames) return launch_mb_bwd_k<F16, D, DV, LAST, true, true, 2>(p, s);
+      return launch_mb_bwd_k<F16, D, DV, LAST, true, false, 2>(p, s);
     }
   }
-  return launch_mb_bwd_k<F16, D, DV, LAST, false, false>(p, s);
+  if constexpr (!TWO_OK)
+    if (p.m <= 64) return launch_mb_bwd_k<F16, D, DV, LAST, false, false, 2>(p, s);
+  if (p.m <= 96) return launch_mb_bwd_k<F16, D, DV, LAST, false, false, 3>(p, s);
+  return launch_mb_bwd_k<F16, D, DV, LAST, false, false, 4>(p, s);
 }
 
 template <bool F16>

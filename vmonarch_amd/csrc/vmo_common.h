@@ -198,8 +198,8 @@ constexpr int tile_w(int w) { return w < 32 ? 32 : w; }
 // of a wave complete in order); the caller makes sure no other wave still uses that LDS.  Used by the
 // flash-entropy forward (o) and backward (gradients) and both L-step kernels (u / z, gradients).
 // kEpiPatchBytes is the 32-row patch.  CW = 16: each accumulator block holds 16 valid columns (rows 0-15 of the transposed accumulator; the 16-wide
-// heads, whose LDS tiles hold every row twice), stored as columns 16 a .. 16 a + 15.  PROWS = 16: a 2 KB patch
-// that takes the 32 rows in two halves (for kernels whose LDS budget is that tight).
+// heads, whose LDS tiles hold every row twice), stored as columns 16 a .. 16 a + 15.  PROWS = 16 (8): a 2 KB
+// (1 KB) patch that takes the 32 rows in two (four) parts (for kernels whose LDS budget is that tight).
 constexpr int kEpiPatchBytes = 32 * 32 * 4;
 template <bool F16, int CW = 32, int PROWS = 32>
 __device__ __forceinline__ void store_acc_rows(VMO_LDS float* patch, const f32x16* acc, int nacc, float f, int mode,
@@ -211,7 +211,7 @@ __device__ __forceinline__ void store_acc_rows(VMO_LDS float* patch, const f32x1
   using V8 = typename Elem<F16>::V8;
   const int hl = lane >> 5, l32 = lane & 31, rr0 = lane >> 3, c = lane & 7;
   static_assert(CW == 16 || CW == 32, "block width");
-  static_assert(PROWS == 16 || PROWS == 32, "patch rows");
+  static_assert(PROWS == 8 || PROWS == 16 || PROWS == 32, "patch rows");
   if (CW == 32 && PROWS == 32 && mode == kGradStore && nacc % 2 == 0) {
     // 16-bit rows: two blocks (64 columns) per pass, so that 8 lanes write a whole 128-byte segment
     VMO_LDS char* pb = (VMO_LDS char*)patch;   // [32 rows][8 chunks of 16 bytes], chunk ^ (row & 7)
