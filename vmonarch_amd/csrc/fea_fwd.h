@@ -56,10 +56,15 @@ constexpr int fwd_stage_bytes() {
 __host__ __device__ constexpr int fp8_dim_pos(int d) { return 64 * (d / 64) + 32 * ((d / 8) % 2) + 8 * ((d / 16) % 4) + d % 8; }
 constexpr float kFp8Max = 448.f;   // e4m3's largest finite value (the conversion does not saturate: beyond it is NaN)
 
-// LDS ring slots per workgroup: prefetch two tiles ahead when three slots fit the workgroup's share
-// of the CU's 160 KB (two 4-wave workgroups or one 8-wave workgroup per CU), else one ahead.
+// LDS ring slots per workgroup: prefetch two tiles ahead when three slots stay within 64 KB (and with it within the
+// workgroup's share of the CU's 160 KB), else one ahead.  The key loop reads every slot at compile-time offsets from
+// shared per-lane addresses, and a read's offset field is 16 bits: three 24 KB slots (64-wide q / k with 128-wide
+// values, 128 with 64) took a second set of addresses, which cost the online-entropy variants their second workgroup
+// per CU (64 / 128: spills, so one; now 229 registers) or spills (128 / 64: 13, now none).  64 / 128, fp16, us at three
+// slots and one workgroup per CU -> two and two: 48 heads x 777 tokens 34.3 -> 24.8, 24 x 8192 793 -> 647; 32 / 64, bf16,
+// 12 x 4096 110 -> 77; 128 / 64, 48 x 777 26.1 -> 24.3.
 constexpr int fwd_slots(int stage_bytes, int waves) {
-  return 3 * stage_bytes <= (waves == kFwdWavesLarge ? 160 : 80) * 1024 ? 3 : 2;
+  return 3 * stage_bytes <= 64 * 1024 ? 3 : 2;
 }
 
 // Copies of ROWS-row tiles (kFwdBN, one pipeline stage of the 128-query kernel) of a row-major (token, W) tensor into swizzled LDS tiles.  Wave

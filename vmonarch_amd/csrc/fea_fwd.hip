@@ -31,12 +31,12 @@
 namespace vmo {
 
 // Workgroups per CU the register budget is sized for: a 256-wide value tensor (its accumulators alone are
-// 128 registers), 256-wide q/k heads, and two narrower shapes that spilled inside the key loop at two
-// workgroups per CU (64-wide q/k with 128-wide values and the online entropy; [k | v] with v narrower
+// 128 registers), 256-wide q/k heads, and two narrower shapes that spill inside the key loop at two
+// workgroups per CU (128-wide values over 16- or 32-wide q/k with the online entropy; [k | v] with v narrower
 // than k) run one 4-wave workgroup per CU.
 template <int D, int DW0, int DW1, int ENT, int WAVES>
 constexpr int fwd_min_blocks() {
-  return (D >= 256 || DW0 >= 256 || (ENT == kEntOnline && tile_w(D) < DW0) || (DW1 > 0 && DW1 < D)) ? 1 : 8 / WAVES;
+  return (D >= 256 || DW0 >= 256 || (ENT == kEntOnline && 4 * tile_w(D) <= DW0) || (DW1 > 0 && DW1 < D)) ? 1 : 8 / WAVES;
 }
 
 // One workgroup's tile, logical index L.
