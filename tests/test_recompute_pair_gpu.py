@@ -38,3 +38,5 @@ def test_recompute_plan():
     assert _recompute_plan(1, 12, 32760, 128, 128, 2, 1560) == (_OVERLAPS["with_r0"], 2)
     assert _recompute_plan(1, 2, 256, 64, 64, 1, 64)[0] == _OVERLAPS["off"]         # values [k | v]: no pair
     assert _recompute_plan(1, 12, 32760, 32, 32, 2, 1560)[0] == _OVERLAPS["start"]   # 32-wide heads: no pair
+    fp8 = _recompute_plan(1, 12, 32760, 128, 128, 2, 1560, qk_fp8=True)              # R-step 0 with fp8 S: no pair
+    assert fp8 == (_OVERLAPS["start"], 3)

@@ -63,13 +63,13 @@ def _recompute_splits(problems, nq, nk, paired=False):
     return max(1, min(16, want, nk // 512))
 
 
-def _recompute_plan(B, H, N, D, Dv, num_iters, rt):
+def _recompute_plan(B, H, N, D, Dv, num_iters, rt, qk_fp8=False):
     """(order, key splits) of the exact recompute of the first rt queries; see _RECOMPUTE_OVERLAP."""
     order = _RECOMPUTE_OVERLAP
     if rt <= 0:
         return 0, 1
     if order == "auto":
-        if num_iters > 1 and D == Dv and D in (64, 128):
+        if num_iters > 1 and D == Dv and D in (64, 128) and not qk_fp8:
             order = "with_r0"
         else:
             order = "start" if 2.0 * B * H * rt * N * (D + Dv) >= _FORK_MIN_FLOPS else "off"
@@ -159,7 +159,7 @@ def _fused_supported(q, k, v, num_blocks):
 # Where the exact recompute of the first rt queries runs: it reads q, k, v only and writes rows [0, rt) of z, which
 # the L-steps never write, so it can run beside the R/L chain.  "with_r0": its workgroups in one launch with R-step
 # 0's; "start" / "after_r0" / "after_r1": on a second stream, forked there and joined at the end; "off": after the
-# chain; "auto": with_r0 where that launch is built (more than one iteration, equal head dims of 64 or 128),
+# chain; "auto": with_r0 where that launch is built (more than one iteration, equal head dims of 64 or 128, no fp8 S),
 # otherwise start from _FORK_MIN_FLOPS on, else off.  Fork and join cost ~45 us of host time in the HIP runtime
 # (event records and cross-stream waits), which small calls waited for; the shared launch costs none.  Whole
 # forward, us, start / off / with_r0: 4 x 64 grid, 2 heads 59.8 / 25.7 / 21.2; 16 x 256, 8 problems 66.8 / 67.4 / 57.7;
@@ -188,7 +188,7 @@ def _vmonarch_fused(q, k, v, m, b, num_iters, recompute_tokens, min_col_mass, st
     B, H, N, D = q.shape
     scale = D ** -0.5 if scale is None else scale
     rt = min(int(recompute_tokens), N)
-    overlap, splits = _recompute_plan(B, H, N, D, v.shape[-1], num_iters, rt)
+    overlap, splits = _recompute_plan(B, H, N, D, v.shape[-1], num_iters, rt, qk_fp8)
     side = _side_stream(q.device) if overlap not in (0, 4) else None
     main = torch.cuda.current_stream(q.device) if stage_hook is not None else None
     return _lib.host().vmonarch_fwd(q, k, v, m, b, num_iters, rt, min_col_mass, scale, qk_fp8, splits, overlap,
