@@ -251,7 +251,8 @@ typedef struct vmo_lstep_bwd_args {
   /* Optional (null: not written): delta[token] = sum_f out[token][f] * grad_out[token][f] in fp32 over the
    * 16-bit values as stored, (B, H, m*b) with token stride 1 -- the per-row sum the flash-entropy backward of
    * the R-step that produced `out` needs (vmo_fea_bwd_args.delta), formed here from rows this kernel holds
-   * anyway.  Built for the one-tile kernels (m <= 32, d and dv in {64, 128}); other shapes reject it. */
+   * anyway.  Built for the one-tile kernels (m <= 32, d and dv in {64, 128}), and through
+   * vmo_lstep_bwd_delta for the multi-block ones' last step; other shapes reject it. */
   float* delta;
   int64_t delta_stride_b, delta_stride_h;
 } vmo_lstep_bwd_args;
@@ -307,6 +308,10 @@ int vmo_lstep_fwd(const vmo_lstep_args* args, void* stream);
 
 /* Backward of the fused L-step; see vmo_lstep_bwd_args. */
 int vmo_lstep_bwd(const vmo_lstep_bwd_args* args, void* stream);
+
+/* vmo_lstep_bwd, with `delta` also from the last step of the multi-block grids (m <= 128 and head dims 16 / 32 / 64 /
+ * 128); their other steps and the general kernel's shapes reject it. */
+int vmo_lstep_bwd_delta(const vmo_lstep_bwd_args* args, void* stream);
 
 #ifdef __cplusplus
 }

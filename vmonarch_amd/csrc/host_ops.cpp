@@ -280,7 +280,7 @@ void lstep_bwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tens
     a.delta = delta->data_ptr<float>();
     a.delta_stride_b = delta->stride(0); a.delta_stride_h = delta->stride(1);
   }
-  check(vmo_lstep_bwd(&a, stream_of(q)), "vmo_lstep_bwd");
+  check(delta ? vmo_lstep_bwd_delta(&a, stream_of(q)) : vmo_lstep_bwd(&a, stream_of(q)), "vmo_lstep_bwd");
 }
 
 // ---- flash-entropy attention (all N rows valid, head dims the kernels take as they are) --------------------------
@@ -449,6 +449,9 @@ std::tuple<std::vector<int>, std::vector<Tensor>> vmonarch_fwd_train(const Tenso
   return {orders, all};
 }
 
+// Which L-steps' backward kernels form delta: one-tile grids every one, multi-block grids the last.
+enum Delta { kNoDelta = 0, kEveryStep = 1, kLastStep = 2 };
+
 // Call order: the L- and R-step backwards from the last iteration down, R-step 0's last of all and the recompute's
 // (rows [0, rt), vmonarch.py:66-68) just before it.  Every gradient is written once, in the caller's dtype and
 // memory order, by the last call that contributes to it: the fp32 sum of the earlier contributions plus its own
@@ -458,7 +461,7 @@ std::tuple<std::vector<int>, std::vector<Tensor>> vmonarch_fwd_train(const Tenso
 // last R-step (values [k | v]) and the recompute.
 std::tuple<Tensor, Tensor, Tensor> vmonarch_bwd(const std::vector<int>& orders, const std::vector<Tensor>& all, const Tensor& dz0,
                                                 int64_t m, int64_t b, int64_t iters, int64_t rt, double min_col_mass,
-                                                double scale, bool want_delta) {
+                                                double scale, int want_delta) {
   const Tensor &q = all[0], &k = all[1], &v = all[2], &z = all[3], &lse_rt = all[4];
   const Tensor dz = row_aligned(dz0.to(q.scalar_type()));
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Dv = v.size(3);
@@ -476,7 +479,7 @@ std::tuple<Tensor, Tensor, Tensor> vmonarch_bwd(const std::vector<int>& orders, 
   // rowsum(out * d out), formed by the L-step backward that writes d out and read by the R-step backward in place of
   // another pass over both
   OptT delta;
-  if (want_delta) delta = at::empty({B, H, N}, f32(q));
+  if (want_delta != kNoDelta) delta = at::empty({B, H, N}, f32(q));
   // where one call puts its part of a gradient: into the fp32 partial sum (the first call overwrites it), or from
   // its last contribution into the result
   struct Put { const Tensor* g; const Tensor* base; int32_t flags; };
@@ -493,6 +496,7 @@ std::tuple<Tensor, Tensor, Tensor> vmonarch_bwd(const std::vector<int>& orders, 
     const bool last = it == iters - 1;
     const Tensor &x = all[5 + 4 * it], &out = all[6 + 4 * it], &lse = all[7 + 4 * it], &ent = all[8 + 4 * it];
     Tensor dout = at::empty_like(out);
+    if (!last && want_delta != kEveryStep) delta.reset();
     lstep_bwd(q, out, ent, g, dq, dout, m, b, scale, last, last ? rt : 0, min_col_mass, last, delta);
     if (it == 0 && rt > 0) {   // the exact attention of the first rt queries; it reads every key and value
       const Tensor zeros = de.narrow(2, 0, rt);

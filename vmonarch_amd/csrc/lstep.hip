@@ -477,28 +477,15 @@ __global__ __launch_bounds__(64 * kLBWaves, 2) void lstep_bwd_kernel(LBParams p)
   T* const dcol = (T*)p.dout + bb * p.do_sb + hh * p.do_sh + (int64_t)j * p.do_sn;
   const int64_t do_rs = (int64_t)p.bs * p.do_sn;
 
-  // delta_k = sum_f out[k][f] d out[k][f] (p.delta): d out's accumulator blocks (lane (k, hl): features 32 a +
-  // 8 g + 4 hl + 0..3), rounded as they are stored, against out's row k held as MFMA operands (features
-  // 16 ds + 8 hl + 0..7).  Two permlane32 swaps per operand trade the middle 4-feature groups between the
-  // halves, so that lane (k, hl) holds features 16 ds + 4 hl + 0..3 (X) and 16 ds + 8 + 4 hl + 0..3 (Y):
-  // groups g = 2 (ds % 2) and 2 (ds % 2) + 1 of block ds / 2.
+  // delta_k = sum_f out[k][f] d out[k][f] (p.delta): out's row k held as MFMA operands against d out's accumulators
   auto row_dot = [&](const V8* rowf, const f32x16* acc, auto nblocks_tag) __attribute__((always_inline)) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    using V2 = typename E::V2;
     float d = 0.f;
 #pragma unroll
     for (int ds = 0; ds < 2 * decltype(nblocks_tag)::value; ++ds) {
-      const u32x4 w = __builtin_bit_cast(u32x4, rowf[ds]);
-      const auto s0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
-      const auto s1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
-      const uint32_t xy[4] = {s0[0], s1[0], s0[1], s1[1]};   // X: accumulator rows r0 .. r0+3, Y: r0+4 .. r0+7
-      const int r0 = 8 * (ds & 1);
+      V8 x;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const V2 x = __builtin_bit_cast(V2, xy[u]);
-        d = fmaf((float)to_elem<T>(acc[ds >> 1][r0 + 2 * u]), (float)x[0], d);
-        d = fmaf((float)to_elem<T>(acc[ds >> 1][r0 + 2 * u + 1]), (float)x[1], d);
-      }
+      for (int e = 0; e < 8; ++e) x[e] = to_elem<T>(acc[ds >> 1][8 * (ds & 1) + e]);
+      d = row_dot16<F16>(rowf[ds], x, d);
     }
     return d;
   };
@@ -1058,9 +1045,10 @@ extern "C" int vmo_lstep_fwd(const vmo_lstep_args* a, void* stream) {
 }
 
 
-extern "C" int vmo_lstep_bwd(const vmo_lstep_bwd_args* a, void* stream) {
-  using namespace vmo;
-  clear_error();
+namespace vmo {
+
+// any_delta: delta on the multi-block grids' last step too (vmo_lstep_bwd_delta)
+static int lstep_bwd_impl(const vmo_lstep_bwd_args* a, void* stream, bool any_delta) {
   if (!a) return set_error(VMO_ERR_INVALID, "lstep_bwd: null args");
   if (a->dtype != VMO_DTYPE_BF16 && a->dtype != VMO_DTYPE_F16) return set_error(VMO_ERR_INVALID, "lstep_bwd: dtype");
   if (a->batch < 0 || a->heads < 0 || a->num_blocks < 1 || a->block_size < 1)
@@ -1081,7 +1069,7 @@ extern "C" int vmo_lstep_bwd(const vmo_lstep_bwd_args* a, void* stream) {
   if (cols > (1ll << 30) || (int64_t)a->num_blocks * a->block_size > (1ll << 30))
     return set_error(VMO_ERR_UNSUPPORTED, "lstep_bwd: problem too large");
   if (a->flags & ~VMO_LSTEP_BWD_OVERWRITE_Q) return set_error(VMO_ERR_INVALID, "lstep_bwd: unknown flags 0x%x", (unsigned)a->flags);
-  if (a->delta && !one_tile)
+  if (a->delta && !one_tile && !(any_delta && multi_block && a->last))
     return set_error(VMO_ERR_UNSUPPORTED, "lstep_bwd: delta is built for the one-tile kernels (m <= 32, d and dv in "
                      "{64, 128}); got m=%d d=%d dv=%d", a->num_blocks, a->d, a->dv);
   LBParams p{};
@@ -1115,4 +1103,16 @@ extern "C" int vmo_lstep_bwd(const vmo_lstep_bwd_args* a, void* stream) {
   }
   if (a->dtype == VMO_DTYPE_F16) return dispatch_lstep_bwd<true>(p, a->d, a->dv, a->last != 0, s);
   return dispatch_lstep_bwd<false>(p, a->d, a->dv, a->last != 0, s);
+}
+
+}  // namespace vmo
+
+extern "C" int vmo_lstep_bwd(const vmo_lstep_bwd_args* a, void* stream) {
+  vmo::clear_error();
+  return vmo::lstep_bwd_impl(a, stream, false);
+}
+
+extern "C" int vmo_lstep_bwd_delta(const vmo_lstep_bwd_args* a, void* stream) {
+  vmo::clear_error();
+  return vmo::lstep_bwd_impl(a, stream, true);
 }

@@ -712,6 +712,23 @@ __global__ __launch_bounds__(64 * kMbWaves, (mb_bwd_min_waves<D, DV, LAST, TWO, 
         asm volatile("" ::: "memory");
       }
   };
+  // p.delta: delta_k = sum_f out[k][f] d out[k][f] of this lane's key, from d out's accumulator blocks as stored and
+  // out's row k as operands row(ds) (features 16 ds + 8 hl ..): this half's part.  Formed here it costs those operand
+  // reads; the R-step backward's own pass read all of out and d out again.  96 x 341, 12 heads: that pass 100 -> 5 us, this
+  // kernel 189 -> 227, the training step 2393 -> 2332; 48 x 211, 8 heads, 64-wide (three steps) 326 -> 317.  Last step
+  // only: the other steps' kernel has no registers to spare (156 and more spilled).
+  auto row_dot = [&](const auto& acc, auto n_tag, auto row, float d) __attribute__((always_inline)) {
+    constexpr int N = decltype(n_tag)::value;
+#pragma unroll
+    for (int ds = 0; ds < N; ++ds) d = row_dot16<F16>(row(ds), mb_pack<T, V8>(acc[ds / 2], ds % 2, 1.f), d);
+    return d;
+  };
+  float* delta = nullptr;   // in scalar registers: kept through every pass
+  if (p.delta) {
+    const uint64_t u = (uint64_t)(uintptr_t)(p.delta + bb * p.dl_sb + hh * p.dl_sh + j);
+    delta = (float*)(uintptr_t)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(u >> 32)) << 32 |
+                                (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)u));
+  }
   // The two-block kernels (TWO) give each wave a (query block ib, key block kb) pair.  pair_lse: the row LSE of
   // the query rows from the S^T blocks of the pairs (each wave's x), as the partial max and sum of each key
   // block combined through `part` (rows past m get +1e30: their attention is exactly zero).  pair_row_sum: a
@@ -742,6 +759,15 @@ __global__ __launch_bounds__(64 * kMbWaves, (mb_bwd_min_waves<D, DV, LAST, TWO, 
     if (hl == 0) part[kb * M + 32 * ib + l32] = v;
     __syncthreads();
     return part[32 * ib + l32] + part[M + 32 * ib + l32];
+  };
+
+  // delta from the two column halves' partials (between two barriers: after the first the sums are read)
+  auto put_pair_delta = [&](float d, int half, int kq) __attribute__((always_inline)) {
+    d = wave_sum32(d);
+    if (hl == 0) part[half * M + 32 * kq + l32] = d;
+  };
+  auto store_pair_delta = [&]() __attribute__((always_inline)) {
+    if (tid < m) delta[(int64_t)tid * p.bs] = part[tid] + part[M + tid];
   };
 
   // One-block-per-wave passes.  put_mat: this wave's block row (lane: row l32 of block blk, accumulator order over
@@ -880,7 +906,14 @@ __global__ __launch_bounds__(64 * kMbWaves, (mb_bwd_min_waves<D, DV, LAST, TWO, 
             acck[a] = E::mfma(mb_tr8<V8, RBD, CT>(q_t, i2, m, lane, iq * NH + a, 1), P1, acck[a]);
           }
         }
+        if (delta) {
+          auto y_row = [&](int ds) { return mb_row8<V8, RBY, CT>(y_t, kq, m, l32, hl, 2 * iq * NVH + ds); };
+          auto k_row = [&](int ds) { return mb_row8<V8, RBD, CT>(k_t, kq, m, l32, hl, 2 * iq * NH + ds); };
+          put_pair_delta(row_dot(acck, std::integral_constant<int, 2 * NH>{}, k_row,
+                                 row_dot(accy, std::integral_constant<int, 2 * NVH>{}, y_row, 0.f)), iq, kq);
+        }
         __syncthreads();
+        if (delta) store_pair_delta();
         const int nr = min(32, m - 32 * kq);
         store_rows(std::integral_constant<int, CWV>{}, accy, NVH, kGradStore,
                    (char*)(dcol + 32 * kq * do_rs + D + 32 * iq * NVH), do_rs * 2, nr);
@@ -943,9 +976,20 @@ __global__ __launch_bounds__(64 * kMbWaves, (mb_bwd_min_waves<D, DV, LAST, TWO, 
         put_rows(g_t, std::integral_constant<int, RBG>{}, g_rows, NDSV);
       }
       __syncthreads();
+      // out's row of this lane's key, read again (kr and y are overlaid by now) beside the products
+      auto load_out = [&](auto& row, int col0) __attribute__((always_inline)) {
+        const T* const src = ocol + (int64_t)min(32 * blk + l32, m - 1) * o_rs + 8 * hl + col0;
+        constexpr int N = sizeof(row) / sizeof(V8);
+#pragma unroll
+        for (int ds = 0; ds < N; ++ds) row[ds] = *(const V8*)(src + 16 * ds);
+      };
+      float dlt = 0.f;
       if (busy) {   // dy^T[dv][k] += sum_i g^T[dv][i] a[i][k]
         f32x16 accy[NV];
+        V8 y_row[NDSV];
+        if (delta) load_out(y_row, D);
         mat_product(accy, std::integral_constant<int, NV>{}, std::integral_constant<int, RBG>{}, g_t, sm + Lo.mat0, true);
+        if (delta) dlt = row_dot(accy, std::integral_constant<int, NDSV>{}, [&](int ds) { return y_row[ds]; }, 0.f);
         store_rows(std::integral_constant<int, CWV>{}, accy, NV, kGradStore, (char*)(dcol + 32 * blk * do_rs + D),
                    do_rs * 2, nrows);
       }
@@ -957,7 +1001,13 @@ __global__ __launch_bounds__(64 * kMbWaves, (mb_bwd_min_waves<D, DV, LAST, TWO, 
       __syncthreads();
       if (busy) {   // dkr^T[d][k] += sum_i q^T[d][i] dl[i][k]
         f32x16 acck[ND];
+        V8 k_row[NDS];
+        if (delta) load_out(k_row, 0);
         mat_product(acck, std::integral_constant<int, ND>{}, std::integral_constant<int, RBD>{}, q_t, sm + Lo.mat1, true);
+        if (delta) {
+          dlt = wave_sum32(row_dot(acck, std::integral_constant<int, NDS>{}, [&](int ds) { return k_row[ds]; }, dlt));
+          if (row_ok && hl == 0) delta[(int64_t)(32 * blk + l32) * p.bs] = dlt;
+        }
         store_rows(std::integral_constant<int, CWD>{}, acck, ND, kGradStore, (char*)(dcol + 32 * blk * do_rs), do_rs * 2,
                    nrows);
       }

@@ -44,7 +44,7 @@ struct LBParams {
   float logit_scale_log2;
   float scale;
   float min_col_mass;
-  float* delta;       // optional: sum_f out * d out per token (one-tile kernels)
+  float* delta;       // optional: sum_f out * d out per token (one-tile kernels, multi-block last step)
   int64_t dl_sb, dl_sh;
 };
 

@@ -174,6 +174,28 @@ __device__ __forceinline__ V8 lds_read_tr8(const VMO_LDS char* p0, const VMO_LDS
 template <class T>
 __device__ __forceinline__ T to_elem(float x) { return static_cast<T>(x); }
 
+// d + the dot product of 16 features of an output row: x, a row operand (lane (row l32, half hl): features 16 ds +
+// 8 hl + 0..7), against y, accumulator rows 8 (ds % 2) .. + 7 of block ds / 2 of the transposed result, rounded as they are
+// stored (lane (l32, hl): features 16 ds + 4 hl + 0..3, then 16 ds + 8 + 4 hl + 0..3).  Two permlane32 swaps trade x's
+// middle 4-feature groups between the halves.  The two halves' sums add to the row's.
+template <bool F16>
+__device__ __forceinline__ float row_dot16(typename Elem<F16>::V8 x, typename Elem<F16>::V8 y, float d) {
+  using V2 = typename Elem<F16>::V2;
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const u32x4 w = __builtin_bit_cast(u32x4, x), z = __builtin_bit_cast(u32x4, y);
+  const auto s0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+  const auto s1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+  const uint32_t xy[4] = {s0[0], s1[0], s0[1], s1[1]};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const uint32_t zu = z[u];   // (a vector element cannot be cast in place: that reads element 0)
+    const V2 a = __builtin_bit_cast(V2, zu), v = __builtin_bit_cast(V2, xy[u]);
+    d = fmaf((float)a[0], (float)v[0], d);
+    d = fmaf((float)a[1], (float)v[1], d);
+  }
+  return d;
+}
+
 // How a result row is written: in the inputs' 16-bit type, into an fp32 buffer (added to or
 // overwritten), or in the 16-bit type as the sum with an fp32 base row (the last of several
 // contributions to one gradient).

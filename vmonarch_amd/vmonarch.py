@@ -88,7 +88,7 @@ def _lstep_one_tile(m, d, dv, last):
 def _lstep_bwd_launch(q, out, ent, grad_res, grad_q, grad_out, m, b, scale, last, skip, min_col_mass,
                       overwrite_q=False, delta=None):
     """Backward of one L-step (vmo_lstep_bwd): grad_q (fp32) += dL/dq (= with overwrite_q),
-    grad_out = dL/d out; with `delta` ((B, H, N) fp32, one-tile grids only) also rowsum(out * grad_out)."""
+    grad_out = dL/d out; with `delta` ((B, H, N) fp32; one-tile grids, and multi-block ones' last step) also rowsum(out * grad_out)."""
     _lib.host().lstep_bwd(q, out, ent, grad_res, grad_q, grad_out, m, b, scale, bool(last), skip, min_col_mass,
                           bool(overwrite_q), delta)
 
@@ -231,8 +231,8 @@ class _VMonarchFunction(torch.autograd.Function):
         m, b, num_iters, rt, min_col_mass, scale = ctx.dims
         saved = ctx.saved_tensors
         D, Dv = saved[0].shape[-1], saved[2].shape[-1]
-        grads = _lib.host().vmonarch_bwd(ctx.orders, saved, dz, m, b, num_iters, rt, min_col_mass, scale,
-                                         _lstep_one_tile(m, D, Dv, True))
+        delta = 1 if _lstep_one_tile(m, D, Dv, True) else 2 if _lstep_mb(m, D, Dv, True) else 0   # (enum Delta)
+        grads = _lib.host().vmonarch_bwd(ctx.orders, saved, dz, m, b, num_iters, rt, min_col_mass, scale, delta)
         return *grads, None, None, None, None, None, None
 
 
