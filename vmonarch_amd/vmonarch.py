@@ -53,13 +53,17 @@ def _recompute_splits(problems, nq, nk, paired=False):
     On its own: the fewest that fill ~80% of one round of workgroup slots (two 128-query workgroups per CU), each
     split keeping >= 512 keys (measured at cfg4, 156 query tiles: 3 splits 0.300 ms, 8 splits 0.309, 16 splits 0.336).
     In one launch with R-step 0, whose workgroups fill the other slots: the fewest that make 120 workgroups, at least
-    two (one workgroup walking all keys would outlast the R-step) and at most eight, each of >= 256 keys.  Measured,
-    whole forward in us at 2 / 4 / 8 / 16 splits: 16 query tiles x 4096 keys 75.9 / 64.6 / 61.0 / 65.4; 24 x 4200 88.2 /
-    76.1 / 81.9 / 85.1; 48 x 13200 279 / 255 / 261 / 271; 156 x 32760 1209 / 1215 / 1237 / 1269 (1 split: 1236)."""
+    two (one workgroup walking all keys would outlast the R-step) until the recompute's tiles fill a round by themselves
+    (the line of the rule above, 409 tiles; from there a second split only writes and merges partials), and at most
+    eight, each of >= 256 keys.  Measured, whole forward in us at 2 / 4 / 8 / 16 splits: 16 query tiles x 4096 keys
+    75.9 / 64.6 / 61.0 / 65.4; 24 x 4200 88.2 / 76.1 / 81.9 / 85.1; 48 x 13200 279 / 255 / 261 / 271; 156 x 32760
+    1209 / 1215 / 1237 / 1269.  At 1 / 2 splits: 156 x 32760 1190 / 1153; 252 x 32760 1301 / 1313; 312 x 32760 1441 /
+    1429; 624 x 32760 4530 / 4557; 732 x 32760 2164 / 2193; 3072 x 32760 (all tokens) 6277 / 6420, and 406 MB of
+    partials."""
     base = problems * ((nq + 127) // 128)
-    if paired:
-        return max(1, min(8, max(2, -(-120 // base)), nk // 256))
     want = -(-int(0.8 * 2 * _NUM_CUS) // base)
+    if paired:
+        return max(1, min(8, max(min(2, want), -(-120 // base)), nk // 256))
     return max(1, min(16, want, nk // 512))
 
 
