@@ -9,3 +9,22 @@ import pytest
 def test_paired_recompute_is_not_split_once_its_tiles_fill_the_chip(B, H, m, b, rt, splits):
     from vmonarch_amd.vmonarch import _OVERLAPS, _recompute_plan
     assert _recompute_plan(B, H, m * b, 128, 128, 2, rt) == (_OVERLAPS["with_r0"], splits)
+
+
+def test_calls_that_something_records_take_the_autograd_function():
+    import torch
+    from vmonarch_amd.kernel import _recorded
+    x, leaf, seen = torch.randn(1, 2, 8, 16), torch.randn(1, 2, 8, 16, requires_grad=True), []
+
+    def note(t):
+        seen.append(_recorded(x, t, x))
+        return t * 2
+
+    assert not _recorded(x, x, x) and _recorded(x, x, leaf)
+    with torch.no_grad():
+        assert not _recorded(x, x, leaf)
+        torch.func.vmap(note)(x)
+        with torch.autograd.forward_ad.dual_level():
+            note(x)
+        torch.jit.trace(note, (x,), check_trace=False)
+    assert seen == [True, True, True]

@@ -95,12 +95,18 @@ class _FlashEntropyAttention(torch.autograd.Function):
         return dq, dk, dv, None, None, None
 
 
+def _recorded(*tensors):
+    """Whether something records the call: autograd, a functorch transform, forward-mode AD or torch.jit's tracer (which
+    would see the host module's allocations only)."""
+    return ((torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            or torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None)
+
+
 def _plain_call(q, k, v):
-    """Whether flash_entropy_attention can go straight to the kernels: no gradient or transform to record (autograd's
-    function, ~12 us of host time, is then only passed through), and inputs that its forward takes as they are."""
-    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
-        return False
-    if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
+    """Whether flash_entropy_attention can go straight to the kernels: nothing records the call (autograd's function,
+    ~12 us of host time, is then only passed through), and inputs that its forward takes as they are."""
+    if _recorded(q, k, v):
         return False
     if not (type(q) is type(k) is type(v) is torch.Tensor and q.is_cuda and q.dim() == 4):
         return False
