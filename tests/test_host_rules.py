@@ -28,3 +28,34 @@ def test_calls_that_something_records_take_the_autograd_function():
             note(x)
         torch.jit.trace(note, (x,), check_trace=False)
     assert seen == [True, True, True]
+
+
+@pytest.mark.parametrize("which", ["k", "v"])
+@pytest.mark.parametrize("other", ["float32", "float16", "uint8"])
+def test_inputs_of_another_dtype_are_refused(which, other):
+    """The kernels read every input in q's type: a wider one would be read as other numbers, a narrower one past its end.
+    Refused on the host before any launch, by the public entry and by the host module under it."""
+    import torch
+    from vmonarch_amd import _lib, flash_entropy_attention
+    x = {n: torch.zeros(1, 2, 8, 16, dtype=torch.bfloat16) for n in "qkv"}
+    x[which] = x[which].to(getattr(torch, other))
+    with pytest.raises(AssertionError, match="one dtype"):
+        flash_entropy_attention(**x)
+    host, (q, k, v) = _lib.host(), x.values()
+    for call in (lambda: host.fea_attention(q, k, v, 1.0),
+                 lambda: host.vmonarch_fwd(q, k, v, 2, 4, 2, 0, 0.01, 1.0, False, 1, 0, 0, None, None, None),
+                 lambda: host.vmonarch_fwd_train(q, k, v, 2, 4, 2, 0, 0.01, 1.0, 1, 0, 0)):
+        with pytest.raises(AssertionError, match="dtype"):
+            call()
+
+
+def test_inputs_elsewhere_are_refused():
+    import torch
+    from vmonarch_amd import _lib
+    q, far = torch.zeros(1, 2, 8, 16, dtype=torch.bfloat16), torch.zeros(1, 2, 8, 16, dtype=torch.bfloat16, device="meta")
+    host = _lib.host()
+    for k, v in ((far, q), (q, far)):
+        with pytest.raises(AssertionError, match="device"):
+            host.fea_attention(q, k, v, 1.0)
+    with pytest.raises(ValueError, match="GPU"):
+        host.fea_attention(q, q, q, 1.0)

@@ -17,6 +17,7 @@
 
 #include <algorithm>
 #include <array>
+#include <initializer_list>
 #include <optional>
 #include <string>
 #include <tuple>
@@ -48,6 +49,25 @@ int dtype_code(const Tensor& t) {
   if (t.scalar_type() == at::kBFloat16) return VMO_DTYPE_BF16;
   if (t.scalar_type() == at::kHalf) return VMO_DTYPE_F16;
   raise(PyExc_KeyError, std::string("torch.") + c10::toString(t.scalar_type()));
+}
+
+// The kernels take every tensor's type and place from q, so a tensor of another type would be read as what it is not, and
+// one elsewhere through an address the GPU does not have.
+void on_gpu(const Tensor& q) {
+  if (!q.is_cuda()) raise(PyExc_ValueError, "vmonarch_amd: needs GPU tensors, got " + q.device().str());
+}
+void same_device(const Tensor& q, const Tensor& t) { require(t.device() == q.device(), "all tensors on q's device"); }
+void like(const Tensor& q, const Tensor& t) {
+  require(t.scalar_type() == q.scalar_type(), "all of q's dtype");
+  same_device(q, t);
+}
+void like(const Tensor& q, std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    if (t) like(q, *t);
+}
+void same_device(const Tensor& q, std::initializer_list<const Tensor*> ts) {
+  for (const Tensor* t : ts)
+    if (t) same_device(q, *t);
 }
 
 // (B, H, N, F) tensor -> view (element strides, feature dim contiguous)
@@ -108,6 +128,9 @@ struct FwdCall {
   int64_t rows;
 };
 vmo_fea_fwd_args fwd_args(const FwdCall& c) {
+  on_gpu(c.q);
+  like(c.q, {&c.k, &c.w0, c.w1, &c.o});
+  same_device(c.q, {c.lse, c.ent});
   vmo_fea_fwd_args a{};
   a.dtype = dtype_code(c.q);
   a.batch = c.q.size(0); a.heads = c.q.size(1); a.frames = c.frames;
@@ -182,6 +205,9 @@ struct BwdCall {
   int64_t rows;   // >= 0: only the first `rows` queries
 };
 void run_bwd(const BwdCall& c) {
+  on_gpu(c.q);
+  like(c.q, {&c.k, &c.v, c.v1, &c.o, &c.dO});
+  same_device(c.q, {&c.lse, &c.ent, &c.dE, c.dq, c.dk, c.dv, c.dq_base, c.dk_base, c.dv_base, c.delta});
   vmo_fea_bwd_args a{};
   a.flags = c.flags;
   a.dtype = dtype_code(c.q);
@@ -250,6 +276,9 @@ std::tuple<Tensor, Tensor, OptT> fea_bwd(const Tensor& q, const Tensor& k, const
 
 void lstep_fwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tensor& res, int64_t m, int64_t b, double scale,
                bool last, int64_t skip, double min_col_mass) {
+  on_gpu(q);
+  like(q, {&out, &res});
+  same_device(q, ent);
   vmo_lstep_args a{};
   a.dtype = dtype_code(q);
   a.batch = q.size(0); a.heads = q.size(1); a.num_blocks = m; a.block_size = b;
@@ -265,6 +294,10 @@ void lstep_fwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tens
 void lstep_bwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tensor& grad_res, const Tensor& grad_q,
                const Tensor& grad_out, int64_t m, int64_t b, double scale, bool last, int64_t skip, double min_col_mass,
                bool overwrite_q, const OptT& delta) {
+  on_gpu(q);
+  like(q, {&out, &grad_res, &grad_out});
+  require(grad_q.scalar_type() == at::kFloat, "grad_q: float32");
+  same_device(q, {&ent, &grad_q, ptr(delta)});
   vmo_lstep_bwd_args a{};
   a.dtype = dtype_code(q);
   a.batch = q.size(0); a.heads = q.size(1); a.num_blocks = m; a.block_size = b;
@@ -286,6 +319,8 @@ void lstep_bwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tens
 // ---- flash-entropy attention (all N rows valid, head dims the kernels take as they are) --------------------------
 
 std::tuple<Tensor, Tensor, Tensor> fea_attention(const Tensor& q0, const Tensor& k0, const Tensor& v0, double sm_scale) {
+  like(q0, {&k0, &v0});
+  on_gpu(q0);
   const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0);
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2);
   Tensor o = empty_in_layout(q0, v.size(3));
@@ -297,6 +332,8 @@ std::tuple<Tensor, Tensor, Tensor> fea_attention(const Tensor& q0, const Tensor&
 std::tuple<Tensor, Tensor, Tensor> fea_attention_bwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor& o0,
                                                      const Tensor& lse, const Tensor& ent, const Tensor& do0,
                                                      const Tensor& dE, double sm_scale) {
+  like(q0, {&k0, &v0, &o0, &do0});
+  on_gpu(q0);
   // the gradients in the memory order of the caller's q, k, v
   Tensor dq = empty_in_layout(q0, q0.size(3)), dk = empty_in_layout(k0, k0.size(3)), dv = empty_in_layout(v0, v0.size(3));
   const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0), o = row_aligned(o0), dO = row_aligned(do0);
@@ -348,6 +385,8 @@ struct Stages {   // the caller's stage hook (None: none), with the torch stream
 Tensor vmonarch_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, int64_t m, int64_t b, int64_t iters,
                     int64_t recompute_tokens, double min_col_mass, double scale, bool qk_fp8, int64_t splits, int overlap,
                     int64_t side_handle, py::object hook, py::object main_obj, py::object side_obj) {
+  like(q0, {&k0, &v0});
+  on_gpu(q0);
   const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0);
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Dv = v.size(3);
   const int64_t rt = std::min<int64_t>(recompute_tokens, N);
@@ -403,6 +442,8 @@ std::tuple<std::vector<int>, std::vector<Tensor>> vmonarch_fwd_train(const Tenso
                                                                      int64_t m, int64_t b, int64_t iters, int64_t rt,
                                                                      double min_col_mass, double scale, int64_t splits,
                                                                      int overlap, int64_t side_handle) {
+  like(q0, {&k0, &v0});
+  on_gpu(q0);
   std::vector<int> orders;
   for (const Tensor* t : {&q0, &k0, &v0})
     for (int d : layout_order(*t)) orders.push_back(d);
@@ -463,6 +504,8 @@ std::tuple<Tensor, Tensor, Tensor> vmonarch_bwd(const std::vector<int>& orders, 
                                                 int64_t m, int64_t b, int64_t iters, int64_t rt, double min_col_mass,
                                                 double scale, int want_delta) {
   const Tensor &q = all[0], &k = all[1], &v = all[2], &z = all[3], &lse_rt = all[4];
+  on_gpu(q);
+  same_device(q, dz0);
   const Tensor dz = row_aligned(dz0.to(q.scalar_type()));
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Dv = v.size(3);
   const int64_t dims[3] = {B, H, N};

@@ -54,12 +54,14 @@ class _FlashEntropyAttention(torch.autograd.Function):
         B, H, N, D = q.shape
         Dv = v.shape[-1]
         assert q.dtype in _lib.DTYPES, f"unsupported dtype {q.dtype}"
+        assert k.dtype == v.dtype == q.dtype, f"q, k and v of one dtype, got {q.dtype}, {k.dtype} and {v.dtype}"
         assert k.shape == q.shape and v.shape[:-1] == q.shape[:-1]
         assert D in _HEAD_DIMS and Dv in _HEAD_DIMS
         if D == 256 and Dv != 256:
             raise NotImplementedError("vmonarch_amd: head dim 256 for q/k is built with 256-wide values only")
         if not q.is_cuda:
             raise RuntimeError("vmonarch_amd: flash_entropy_attention needs GPU tensors (no CPU path)")
+        assert k.device == v.device == q.device, f"q, k and v on one GPU, got {q.device}, {k.device} and {v.device}"
         n = int(n_valid)
         Dk, Dvk = _kernel_widths(D, Dv)
         ctx.sm_scale = sm_scale
@@ -111,7 +113,8 @@ def _plain_call(q, k, v):
     if not (type(q) is type(k) is type(v) is torch.Tensor and q.is_cuda and q.dim() == 4):
         return False
     D, Dv = q.shape[-1], v.shape[-1]
-    return (q.dtype in _lib.DTYPES and k.shape == q.shape and v.shape[:-1] == q.shape[:-1] and D in _HEAD_DIMS
+    return (q.dtype in _lib.DTYPES and k.dtype == v.dtype == q.dtype and k.device == v.device == q.device
+            and k.shape == q.shape and v.shape[:-1] == q.shape[:-1] and D in _HEAD_DIMS
             and Dv in _HEAD_DIMS and not (D == 256 and Dv != 256) and _kernel_widths(D, Dv) == (D, Dv))
 
 
