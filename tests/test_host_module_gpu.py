@@ -1,0 +1,68 @@
+"""The host module's manners towards the rest of the program: other Python threads, the caller's device, the stage hook,
+inputs that it must not launch with."""
+import threading
+import time
+
+import pytest
+import torch
+
+from conftest import randn_lp
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _longest_stall(call):
+    """Seconds `call` took and the longest time within it that another Python thread could not run."""
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks.append(time.perf_counter())
+            time.sleep(1e-3)
+
+    th = threading.Thread(target=tick)
+    th.start()
+    time.sleep(0.02)
+    t0 = time.perf_counter()
+    call()
+    t1 = time.perf_counter()
+    time.sleep(0.02)
+    stop.set()
+    th.join()
+    marks = [t for t in ticks if t0 <= t <= t1]
+    return t1 - t0, max(b - a for a, b in zip([t0, *marks], [*marks, t1]))
+
+
+@pytest.mark.parametrize("which", ["attention", "vmonarch", "vmonarch_train"])
+def test_other_threads_run_while_a_call_waits_in_the_driver(which):
+    """A call whose allocation does not fit under the process's limit gives cached memory back first, which waits for the
+    GPU (here some 0.2 s of queued matrix products): other threads go on meanwhile."""
+    from vmonarch_amd import flash_entropy_attention, vmonarch_attention
+    torch.cuda.empty_cache()
+    x = [torch.zeros(1, 9600, 256, 64, device=DEV, dtype=torch.bfloat16) for _ in range(3)]   # 315 MB each
+    if which == "vmonarch_train":
+        x = [t.requires_grad_() for t in x]
+    run = (lambda: flash_entropy_attention(*x)) if which == "attention" else (lambda: vmonarch_attention(*x, 4, 64, 2))
+    a = torch.randn(8192, 8192, device=DEV, dtype=torch.bfloat16)
+    c = torch.empty_like(a)
+    torch.mm(a, a, out=c)
+    run()   # (everything loaded)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    cached = [torch.empty(100 << 20, device=DEV, dtype=torch.uint8) for _ in range(40)]   # each too small for an output
+    del cached
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)
+        for _ in range(300):
+            torch.mm(a, a, out=c)
+        print(f"waiting call: {which}", flush=True)
+        took, stall = _longest_stall(run)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+    print(f"took {took:.3f} s, longest stall {stall:.3f} s", flush=True)
+    assert took > 0.05, "the call did not wait: nothing tested"
+    assert stall < 0.5 * took

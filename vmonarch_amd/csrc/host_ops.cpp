@@ -19,6 +19,7 @@
 #include <array>
 #include <initializer_list>
 #include <optional>
+#include <stdexcept>
 #include <string>
 #include <tuple>
 #include <utility>
@@ -32,29 +33,37 @@ using OptT = std::optional<Tensor>;
 
 namespace {
 
-[[noreturn]] void raise(PyObject* type, const std::string& msg) {
-  PyErr_SetString(type, msg.c_str());
-  throw py::error_already_set();
-}
+// Everything below runs without the interpreter lock, so that other Python threads go on through launches, allocations
+// and whatever waits they lead to in the driver: no Python object is touched, and errors are C++ exceptions that the
+// binding turns into Python's once it holds the lock again.  (std::runtime_error: RuntimeError.)
+struct assertion_error : py::builtin_exception {
+  using builtin_exception::builtin_exception;
+  void set_error() const override { PyErr_SetString(PyExc_AssertionError, what()); }
+};
+struct zero_division_error : py::builtin_exception {
+  using builtin_exception::builtin_exception;
+  void set_error() const override { PyErr_SetString(PyExc_ZeroDivisionError, what()); }
+};
+
 void require(bool ok, const char* msg) {
-  if (!ok) raise(PyExc_AssertionError, msg);
+  if (!ok) throw assertion_error(msg);
 }
 
 void whole_frames(int64_t nq, int64_t nk, int64_t frames) {
-  if (frames == 0) raise(PyExc_ZeroDivisionError, "no frames");
+  if (frames == 0) throw zero_division_error("no frames");
   require(nq % frames == 0 && nk % frames == 0, "whole frames");
 }
 
 int dtype_code(const Tensor& t) {
   if (t.scalar_type() == at::kBFloat16) return VMO_DTYPE_BF16;
   if (t.scalar_type() == at::kHalf) return VMO_DTYPE_F16;
-  raise(PyExc_KeyError, std::string("torch.") + c10::toString(t.scalar_type()));
+  throw py::key_error(std::string("torch.") + c10::toString(t.scalar_type()));
 }
 
 // The kernels take every tensor's type and place from q, so a tensor of another type would be read as what it is not, and
 // one elsewhere through an address the GPU does not have.
 void on_gpu(const Tensor& q) {
-  if (!q.is_cuda()) raise(PyExc_ValueError, "vmonarch_amd: needs GPU tensors, got " + q.device().str());
+  if (!q.is_cuda()) throw py::value_error("vmonarch_amd: needs GPU tensors, got " + q.device().str());
 }
 void same_device(const Tensor& q, const Tensor& t) { require(t.device() == q.device(), "all tensors on q's device"); }
 void like(const Tensor& q, const Tensor& t) {
@@ -109,7 +118,7 @@ void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t
 
 void check(int rc, const char* what) {
   if (rc != 0)
-    raise(PyExc_RuntimeError, std::string(what) + " failed (code " + std::to_string(rc) + "): " + vmo_last_error());
+    throw std::runtime_error(std::string(what) + " failed (code " + std::to_string(rc) + "): " + vmo_last_error());
 }
 
 // ---- single launches -------------------------------------------------------------------------------------------
@@ -351,15 +360,15 @@ struct SideStream {
   SideStream(const SideStream&) = delete;
   ~SideStream() {   // an error between fork and join: joined all the same, before the workspaces are given back
     if (!open) return;
-    try { join(); } catch (py::error_already_set&) {}
+    try { join(); } catch (const std::runtime_error&) {}
   }
   static void order(hipStream_t after, hipStream_t then) {   // work issued to `then` from here on follows `after`'s
     hipEvent_t e;
-    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) raise(PyExc_RuntimeError, "vmonarch: no event");
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) throw std::runtime_error("vmonarch: no event");
     hipError_t rc = hipEventRecord(e, after);
     if (rc == hipSuccess) rc = hipStreamWaitEvent(then, e, 0);
     (void)hipEventDestroy(e);   // (released once the recorded work is done)
-    if (rc != hipSuccess) raise(PyExc_RuntimeError, std::string("vmonarch: stream order: ") + hipGetErrorString(rc));
+    if (rc != hipSuccess) throw std::runtime_error(std::string("vmonarch: stream order: ") + hipGetErrorString(rc));
   }
   void fork() {
     order(main, side);
@@ -375,22 +384,24 @@ struct SideStream {
 // R-step 0 or after the last R-step; or in one launch with R-step 0 (with more than one iteration: its values are k).
 enum Overlap { kOff = 0, kStart = 1, kAfterR0 = 2, kAfterR1 = 3, kWithR0 = 4 };
 
-struct Stages {   // the caller's stage hook (None: none), with the torch stream objects it is told of
+// the caller's stage hook (None: none), with the torch stream objects it is told of; called with the interpreter lock
+struct Stages {
   py::object hook, main, side;
   void operator()(const char* name, int it, const char* phase, bool on_side = false) const {
-    if (!hook.is_none()) hook(it < 0 ? std::string(name) : name + std::to_string(it), phase, on_side ? side : main);
+    if (hook.is_none()) return;
+    const py::gil_scoped_acquire lock;
+    hook(it < 0 ? std::string(name) : name + std::to_string(it), phase, on_side ? side : main);
   }
 };
 
 Tensor vmonarch_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, int64_t m, int64_t b, int64_t iters,
                     int64_t recompute_tokens, double min_col_mass, double scale, bool qk_fp8, int64_t splits, int overlap,
-                    int64_t side_handle, py::object hook, py::object main_obj, py::object side_obj) {
+                    int64_t side_handle, const Stages& stage) {
   like(q0, {&k0, &v0});
   on_gpu(q0);
   const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0);
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Dv = v.size(3);
   const int64_t rt = std::min<int64_t>(recompute_tokens, N);
-  const Stages stage{std::move(hook), std::move(main_obj), std::move(side_obj)};
   void* const main = stream_of(q);
   Tensor ent = at::empty({B, H, N}, f32(q));
   Tensor z = empty_in_layout(q, Dv);   // in the caller's layout
@@ -565,13 +576,20 @@ std::tuple<Tensor, Tensor, Tensor> vmonarch_bwd(const std::vector<int>& orders, 
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
-  mod.def("fea_fwd", &fea_fwd);
-  mod.def("fea_bwd", &fea_bwd);
-  mod.def("lstep_fwd", &lstep_fwd);
-  mod.def("lstep_bwd", &lstep_bwd);
-  mod.def("fea_attention", &fea_attention);
-  mod.def("fea_attention_bwd", &fea_attention_bwd);
-  mod.def("vmonarch_fwd", &vmonarch_fwd);
-  mod.def("vmonarch_fwd_train", &vmonarch_fwd_train);
-  mod.def("vmonarch_bwd", &vmonarch_bwd);
+  using NoGil = py::call_guard<py::gil_scoped_release>;
+  mod.def("fea_fwd", &fea_fwd, NoGil());
+  mod.def("fea_bwd", &fea_bwd, NoGil());
+  mod.def("lstep_fwd", &lstep_fwd, NoGil());
+  mod.def("lstep_bwd", &lstep_bwd, NoGil());
+  mod.def("fea_attention", &fea_attention, NoGil());
+  mod.def("fea_attention_bwd", &fea_attention_bwd, NoGil());
+  mod.def("vmonarch_fwd", [](const Tensor& q, const Tensor& k, const Tensor& v, int64_t m, int64_t b, int64_t iters,
+                             int64_t recompute_tokens, double min_col_mass, double scale, bool qk_fp8, int64_t splits, int overlap,
+                             int64_t side_handle, py::object hook, py::object main, py::object side) {
+    const Stages stage{std::move(hook), std::move(main), std::move(side)};   // (outlives the release of the lock)
+    const py::gil_scoped_release unlocked;
+    return vmonarch_fwd(q, k, v, m, b, iters, recompute_tokens, min_col_mass, scale, qk_fp8, splits, overlap, side_handle, stage);
+  });
+  mod.def("vmonarch_fwd_train", &vmonarch_fwd_train, NoGil());
+  mod.def("vmonarch_bwd", &vmonarch_bwd, NoGil());
 }
