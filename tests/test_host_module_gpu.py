@@ -66,3 +66,47 @@ def test_other_threads_run_while_a_call_waits_in_the_driver(which):
     print(f"took {took:.3f} s, longest stall {stall:.3f} s", flush=True)
     assert took > 0.05, "the call did not wait: nothing tested"
     assert stall < 0.5 * took
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs a second GPU")
+@pytest.mark.parametrize("order", ["with_r0", "start"])
+def test_tensors_on_another_gpu_than_the_current_one(monkeypatch, order):
+    """The launches, the allocations and the fork's events go to the tensors' GPU whichever is current."""
+    import vmonarch_amd.vmonarch as vm
+    monkeypatch.setattr(vm, "_RECOMPUTE_OVERLAP", order)
+    g = torch.Generator().manual_seed(3)
+    x = [randn_lp(g, 1, 2, 256, 64, scale=0.5) for _ in range(3)]
+    out = []
+    for dev in (0, 1):
+        with torch.cuda.device(0):
+            leaves = [t.to(f"cuda:{dev}").requires_grad_() for t in x]
+            o, e = vm.flash_entropy_attention(*leaves)
+            z = vm.vmonarch_attention(*leaves, 4, 64, 2, recompute_tokens=64)
+            grads = torch.autograd.grad(o.float().sum() + e.sum() + z.float().sum(), leaves)
+            assert torch.cuda.current_device() == 0
+            out.append([t.detach().cpu() for t in (o, e, z, *grads)])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
+def test_the_current_gpu_is_left_as_it_was():
+    from vmonarch_amd import flash_entropy_attention
+    before = torch.cuda.current_device()
+    flash_entropy_attention(*(torch.zeros(1, 1, 8, 64, device=DEV, dtype=torch.bfloat16) for _ in range(3)))
+    assert torch.cuda.current_device() == before
+
+
+def test_inputs_off_the_gpu_are_refused_before_a_launch():
+    from vmonarch_amd import _lib, flash_entropy_attention, vmonarch_attention
+    from vmonarch_amd.kernel import fea_forward
+    x, far = torch.zeros(1, 2, 256, 64, device=DEV, dtype=torch.bfloat16), torch.zeros(1, 2, 256, 64, dtype=torch.bfloat16)
+    for k, v in ((far, x), (x, far)):
+        for call in (lambda: flash_entropy_attention(x, k, v), lambda: vmonarch_attention(x, k, v, 4, 64, 2),
+                     lambda: _lib.host().fea_attention(x, k, v, 0.1), lambda: fea_forward(x, k, v, None, 0.1)):
+            with pytest.raises(AssertionError, match="GPU|device"):
+                call()
+    with pytest.raises(ValueError, match="GPU"):
+        fea_forward(far, far, far, None, 0.1)
+    y = x.clone().requires_grad_()
+    with pytest.raises(AssertionError, match="device"):
+        vmonarch_attention(y, far, x, 4, 64, 2)
