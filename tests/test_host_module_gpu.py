@@ -110,3 +110,29 @@ def test_inputs_off_the_gpu_are_refused_before_a_launch():
     y = x.clone().requires_grad_()
     with pytest.raises(AssertionError, match="device"):
         vmonarch_attention(y, far, x, 4, 64, 2)
+
+
+@pytest.mark.parametrize("order", ["auto", "with_r0", "start", "after_r0", "after_r1", "off"])
+def test_the_stage_hook_hears_of_every_stage(monkeypatch, order):
+    """Every stage begins and ends once, the R- and L-steps in turn on the caller's stream, the recompute on whichever it
+    runs; what the hook raises comes out of the call."""
+    import vmonarch_amd.vmonarch as vm
+    monkeypatch.setattr(vm, "_RECOMPUTE_OVERLAP", order)
+    q, k, v = (torch.zeros(1, 2, 256, 64, device=DEV, dtype=torch.bfloat16) for _ in range(3))
+    heard = []
+    with torch.no_grad():
+        vm._vmonarch_fused(q, k, v, 4, 64, 2, 64, 0.01, stage_hook=lambda *a: heard.append(a))
+    main, side = torch.cuda.current_stream(), vm._side_stream(q.device)
+    calls = [(n, p) for n, p, _ in heard]
+    chain = [(f"{s}{i}", p) for i in range(2) for s in ("rstep", "lstep") for p in ("begin", "end")]
+    assert [c for c in calls if c[0] != "recompute"] == chain
+    assert [p for n, p in calls if n == "recompute"] == ["begin", "end"] and len(calls) == len(chain) + 2
+    on = side if order in ("start", "after_r0", "after_r1") else main
+    assert all(st == (on if n == "recompute" else main) for n, _, st in heard)
+    with pytest.raises(ValueError, match="from the hook"):
+        vm._vmonarch_fused(q, k, v, 4, 64, 2, 64, 0.01, stage_hook=lambda n, p, st: _fail() if n == "lstep0" else None)
+    torch.cuda.synchronize()
+
+
+def _fail():
+    raise ValueError("from the hook")

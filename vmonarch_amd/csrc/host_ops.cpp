@@ -431,8 +431,13 @@ Tensor vmonarch_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, int64_
     out = at::empty({B, H, N, D + (last ? Dv : 0)}, q.options());
     stage("rstep", it, "begin");   // iteration 0 folds u = q * scale into the softmax scale
     const FwdCall rstep{it == 0 ? q : u, k, k, last ? &v : nullptr, it == 0 ? scale : 1.0, m, out, nullptr, &ent, 1, qk_fp8, -1};
-    if (with_r0 && it == 0) run_pair(exact_rows, rstep, main);
-    else run_fwd(rstep, main);
+    if (with_r0 && it == 0) {   // one launch, both stages'
+      stage("recompute", -1, "begin");
+      run_pair(exact_rows, rstep, main);
+      stage("recompute", -1, "end");
+    } else {
+      run_fwd(rstep, main);
+    }
     stage("rstep", it, "end");
     if (rt > 0 && !forked && ((overlap == kAfterR0 && it == 0) || (overlap == kAfterR1 && last))) fork();
     stage("lstep", it, "begin");

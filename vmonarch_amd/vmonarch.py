@@ -186,7 +186,8 @@ def _vmonarch_fused(q, k, v, m, b, num_iters, recompute_tokens, min_col_mass, st
                     qk_fp8=False):
     """All-HIP forward.  `stage_hook(name, phase, stream)`, when given, is called on the host right
     before ("begin") and after ("end") each launch group ("rstep0", "lstep0", ..., "recompute") with
-    the stream it goes to -- used by bench.py to bracket every kernel with events.  `scale` overrides
+    the stream it goes to -- used by bench.py to bracket every kernel with events; where the recompute shares R-step
+    0's launch its calls stand inside rstep0's, around the same launch.  `scale` overrides
     D ** -0.5 (q / k zero-padded past their head dim).  `qk_fp8`: the R-steps' S in fp8 (the recompute
     stays exact)."""
     B, H, N, D = q.shape
