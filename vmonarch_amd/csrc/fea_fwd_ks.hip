@@ -13,6 +13,7 @@
 // Layouts, the fixed reference point m (the max of the problem's first 32 keys) with the exact two-pass fallback,
 // the rounding of P and the entropy modes are those of the 128-query kernel: the same p bit for bit, summed in
 // another order.
+#include <atomic>
 #include <type_traits>
 
 #include "fea_fwd.h"
@@ -353,11 +354,11 @@ static int launch_ks(FwdParams p, hipStream_t stream) {
   p.total_wg = p.problems * p.q_tiles;
   auto kern = fea_fwd_ks_kernel<F16, D, DW0, DW1, W0K, ENT, QG, KG>;
   if (LDS > 65536) {
-    static bool done = false;   // attribute is per function; idempotent, so a benign race
-    if (!done) {
+    static std::atomic<bool> done{false};   // the attribute is per function, and setting it again changes nothing
+    if (!done.load(std::memory_order_relaxed)) {
       if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
         return set_error(VMO_ERR_LAUNCH, "fea_fwd_ks: cannot raise the LDS limit to %d bytes", LDS);
-      done = true;
+      done.store(true, std::memory_order_relaxed);
     }
   }
   hipLaunchKernelGGL(kern, dim3(xcd_grid(p.total_wg)), dim3(64 * kKsWaves), LDS, stream, p);
