@@ -313,3 +313,17 @@ def test_fea_fwd_qk_fp8_workspace_and_rejections(L):
     a.w0 = _lib.View(_addr(1 << 20), 128, 128 * 128, 128)   # values that are not k
     assert L.vmo_fea_fwd(ctypes.byref(a), None) == 2
     assert b"qk_fp8" in L.vmo_last_error()
+
+
+def test_lstep_bwd_delta_refusals_name_what_is_built(L):
+    """Multi-block grids form delta in the last step only, and only through vmo_lstep_bwd_delta."""
+    from vmonarch_amd import _lib
+    a = _lib.LstepBwdArgs()
+    a.dtype, a.batch, a.heads, a.num_blocks, a.block_size, a.d, a.dv = 0, 1, 1, 40, 4, 128, 128
+    a.q = a.out = a.grad_res = a.grad_q = a.grad_out = _lib.View(_addr(), 128, 128, 128)
+    a.ent = a.delta = _addr()
+    assert L.vmo_lstep_bwd_delta(ctypes.byref(a), None) == 2
+    assert b"last step" in L.vmo_last_error() and b"last=0" in L.vmo_last_error()
+    a.last = 1
+    assert L.vmo_lstep_bwd(ctypes.byref(a), None) == 2
+    assert b"vmo_lstep_bwd_delta" in L.vmo_last_error()

@@ -1071,7 +1071,9 @@ static int lstep_bwd_impl(const vmo_lstep_bwd_args* a, void* stream, bool any_de
   if (a->flags & ~VMO_LSTEP_BWD_OVERWRITE_Q) return set_error(VMO_ERR_INVALID, "lstep_bwd: unknown flags 0x%x", (unsigned)a->flags);
   if (a->delta && !one_tile && !(any_delta && multi_block && a->last))
     return set_error(VMO_ERR_UNSUPPORTED, "lstep_bwd: delta is built for the one-tile kernels (m <= 32, d and dv in "
-                     "{64, 128}); got m=%d d=%d dv=%d", a->num_blocks, a->d, a->dv);
+                     "{64, 128})%s; got m=%d d=%d dv=%d last=%d",
+                     any_delta ? " and the multi-block kernels' last step (m <= 128)" : ", and by vmo_lstep_bwd_delta for more",
+                     a->num_blocks, a->d, a->dv, a->last != 0);
   LBParams p{};
   p.delta = a->delta;
   p.dl_sb = a->delta_stride_b; p.dl_sh = a->delta_stride_h;
