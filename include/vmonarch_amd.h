@@ -270,6 +270,11 @@ size_t vmo_fea_fwd_workspace_size(const vmo_fea_fwd_args* args);
 /* FlashEntropyAttention forward; see vmo_fea_fwd_args. */
 int vmo_fea_fwd(const vmo_fea_fwd_args* args, void* stream);
 
+/* Queries per workgroup of the kernel that vmo_fea_fwd takes for these arguments (128, or 32 / 64 for launches of few
+ * query tiles); 0 for an empty call or arguments it rejects (which head dims are built is vmo_fea_fwd's to say).
+ * Launches nothing. */
+int vmo_fea_fwd_query_tile(const vmo_fea_fwd_args* args);
+
 /*
  * Two independent forwards, a and b, issued together: results as vmo_fea_fwd(a) and vmo_fea_fwd(b) (neither may
  * read what the other writes).  VMonarch's exact recompute (a: values v, no entropy, any number of splits) and an

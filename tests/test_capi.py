@@ -327,3 +327,15 @@ def test_lstep_bwd_delta_refusals_name_what_is_built(L):
     a.last = 1
     assert L.vmo_lstep_bwd(ctypes.byref(a), None) == 2
     assert b"vmo_lstep_bwd_delta" in L.vmo_last_error()
+
+
+@pytest.mark.parametrize("d, heads, frames, nq, nk, tile", [
+    (64, 2, 1, 1024, 1024, 32), (64, 8, 1, 1024, 512, 32), (64, 8, 1, 1025, 512, 64), (64, 16, 1, 1024, 1024, 64),
+    (64, 16, 1, 1025, 1024, 128), (64, 2, 1, 1024, 511, 128), (128, 4, 1, 1024, 1024, 64), (128, 2, 64, 128, 512, 64),
+    (128, 2, 64, 129, 512, 128), (128, 4, 1, 0, 1024, 0)])
+def test_query_tile_of_a_forward(L, d, heads, frames, nq, nk, tile):
+    """Tiles of 32 (64-wide heads) or 64 queries while at most 256 of them make the launch, and from 512 keys."""
+    from vmonarch_amd import _lib
+    v = lambda off: _lib.View(_addr(off), 128, 128, 128)   # noqa: E731
+    a = _fwd_args(heads=heads, frames=frames, nq=nq, nk=nk, d=d, dw0=d, w0=v(4096), ent=_addr())
+    assert L.vmo_fea_fwd_query_tile(ctypes.byref(a)) == tile

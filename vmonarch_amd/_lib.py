@@ -101,6 +101,8 @@ def lib():
         L.vmo_fea_fwd.argtypes = [ctypes.POINTER(FeaFwdArgs), c_void_p]
         L.vmo_fea_fwd_noalloc.restype = ctypes.c_int
         L.vmo_fea_fwd_noalloc.argtypes = [ctypes.POINTER(FeaFwdArgs), c_void_p]
+        L.vmo_fea_fwd_query_tile.restype = ctypes.c_int
+        L.vmo_fea_fwd_query_tile.argtypes = [ctypes.POINTER(FeaFwdArgs)]
         L.vmo_lstep_fwd.restype = ctypes.c_int
         L.vmo_lstep_fwd.argtypes = [ctypes.POINTER(LstepArgs), c_void_p]
         L.vmo_lstep_bwd.restype = ctypes.c_int

@@ -138,7 +138,8 @@ struct TileCopy {
 enum { kEntNone = 0, kEntOnline = 1, kEntFromPK = 2 };
 
 // The key-group forward kernel (fea_fwd_ks.hip) for launches whose 128-query tiles would leave the chip idle:
-// true when it takes this one, with the launch's status in *rc.
-bool fwd_ks(const FwdParams& p, bool f16, int d, int dw0, int dw1, bool w0k, bool ent, hipStream_t stream, int* rc);
+// true when it takes this one, with the launch's status in *rc.  With `tile` nothing is launched: its queries per workgroup.
+bool fwd_ks(const FwdParams& p, bool f16, int d, int dw0, int dw1, bool w0k, bool ent, hipStream_t stream, int* rc,
+            int* tile = nullptr);
 
 }  // namespace vmo

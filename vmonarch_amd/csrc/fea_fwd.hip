@@ -1037,6 +1037,16 @@ extern "C" int vmo_fea_fwd(const vmo_fea_fwd_args* a, void* stream) {
   return vmo::fea_fwd_impl(a, a ? a->workspace : nullptr, a ? a->workspace_bytes : 0, stream);
 }
 
+extern "C" int vmo_fea_fwd_query_tile(const vmo_fea_fwd_args* a) {
+  using namespace vmo;
+  clear_error();
+  FwdLaunch l;
+  if (fea_fwd_prepare(a, a ? a->workspace : nullptr, a ? a->workspace_bytes : 0, &l) != VMO_OK || l.empty) return 0;
+  int rc = VMO_OK, tile = 32 * kFwdQB * kFwdWavesSmall;
+  if (!l.split && !l.qk8) (void)fwd_ks(l.p, l.f16, l.d, l.dw0, l.dw1, l.w0k, l.ent, nullptr, &rc, &tile);
+  return tile;
+}
+
 extern "C" int vmo_fea_fwd_pair(const vmo_fea_fwd_args* a, const vmo_fea_fwd_args* b, void* stream) {
   using namespace vmo;
   clear_error();

@@ -377,10 +377,11 @@ static int ks_query_blocks(const FwdParams& p, bool eight) {
 }
 
 template <bool F16, int D, int DW0, int DW1, bool W0K, int ENT>
-static bool dispatch_ks(const FwdParams& p, hipStream_t s, int* rc) {
+static bool dispatch_ks(const FwdParams& p, hipStream_t s, int* rc, int* tile) {
   constexpr bool EIGHT = D == 64 && ks_lds_bytes<D, DW0, DW1, W0K, 8>() <= kKsLdsMax;
   const int qg = ks_query_blocks(p, EIGHT);
   if (qg == 0) return false;
+  if (tile) { *tile = 32 * qg; return true; }
   if constexpr (EIGHT)
     if (qg == 1) { *rc = launch_ks<F16, D, DW0, DW1, W0K, ENT, 1>(p, s); return true; }
   *rc = launch_ks<F16, D, DW0, DW1, W0K, ENT, 2>(p, s);
@@ -388,10 +389,10 @@ static bool dispatch_ks(const FwdParams& p, hipStream_t s, int* rc) {
 }
 
 template <bool F16>
-static bool dispatch_ks_dims(const FwdParams& p, int d, int dw0, int dw1, bool w0k, bool ent, hipStream_t s, int* rc) {
+static bool dispatch_ks_dims(const FwdParams& p, int d, int dw0, int dw1, bool w0k, bool ent, hipStream_t s, int* rc, int* tile) {
 #define VMO_KS(D_, DW0_, DW1_, W0K_, ENT_)                                                  \
   if (d == D_ && dw0 == DW0_ && dw1 == DW1_ && w0k == W0K_ && ent == (ENT_ != kEntNone))    \
-    return dispatch_ks<F16, D_, DW0_, DW1_, W0K_, ENT_>(p, s, rc);
+    return dispatch_ks<F16, D_, DW0_, DW1_, W0K_, ENT_>(p, s, rc, tile);
   VMO_KS(64, 64, 0, false, kEntOnline)
   VMO_KS(64, 128, 0, false, kEntOnline)
   VMO_KS(128, 128, 0, false, kEntOnline)
@@ -403,9 +404,9 @@ static bool dispatch_ks_dims(const FwdParams& p, int d, int dw0, int dw1, bool w
   return false;
 }
 
-bool fwd_ks(const FwdParams& p, bool f16, int d, int dw0, int dw1, bool w0k, bool ent, hipStream_t stream, int* rc) {
-  return f16 ? dispatch_ks_dims<true>(p, d, dw0, dw1, w0k, ent, stream, rc)
-             : dispatch_ks_dims<false>(p, d, dw0, dw1, w0k, ent, stream, rc);
+bool fwd_ks(const FwdParams& p, bool f16, int d, int dw0, int dw1, bool w0k, bool ent, hipStream_t stream, int* rc, int* tile) {
+  return f16 ? dispatch_ks_dims<true>(p, d, dw0, dw1, w0k, ent, stream, rc, tile)
+             : dispatch_ks_dims<false>(p, d, dw0, dw1, w0k, ent, stream, rc, tile);
 }
 
 }  // namespace vmo
