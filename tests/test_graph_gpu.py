@@ -63,3 +63,11 @@ def test_flash_entropy_forward_replays_from_a_graph():
             torch.cuda.synchronize()
             assert torch.equal(o, o_ref) and torch.equal(e, e_ref), f"replay {i}"
             _ = run()
+
+
+def test_vmonarch_forward_with_the_recompute_forked_replays_from_a_graph(monkeypatch):
+    """The recompute's second stream joins the capture through the fork's and join's events."""
+    import vmonarch_amd.vmonarch as vm
+    monkeypatch.setattr(vm, "_RECOMPUTE_OVERLAP", "start")
+    test_vmonarch_forward_replays_from_a_graph(21, 120, 128, 120, torch.bfloat16)
+    test_vmonarch_forward_replays_from_a_graph(4, 256, 64, 256, torch.float16)

@@ -59,3 +59,12 @@ def test_inputs_elsewhere_are_refused():
             host.fea_attention(q, k, v, 1.0)
     with pytest.raises(ValueError, match="GPU"):
         host.fea_attention(q, q, q, 1.0)
+
+
+def test_large_64_wide_grids_fork_the_recompute():
+    """The shared launch takes 64-wide R-step 0 its third workgroup per CU; 128-wide heads have two either way."""
+    from vmonarch_amd.vmonarch import _OVERLAPS, _recompute_plan
+    plan = lambda H, m, b, D: _recompute_plan(1, H, m * b, D, D, 2, b)   # noqa: E731
+    assert plan(12, 21, 1560, 64) == (_OVERLAPS["start"], 3) and plan(12, 4, 1560, 64) == (_OVERLAPS["start"], 3)
+    assert plan(12, 4, 600, 64)[0] == plan(8, 4, 1024, 64)[0] == _OVERLAPS["with_r0"]
+    assert plan(12, 21, 1560, 128)[0] == plan(12, 4, 1560, 128)[0] == _OVERLAPS["with_r0"]

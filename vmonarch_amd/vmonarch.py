@@ -73,10 +73,11 @@ def _recompute_plan(B, H, N, D, Dv, num_iters, rt, qk_fp8=False):
     if rt <= 0:
         return 0, 1
     if order == "auto":
-        if num_iters > 1 and D == Dv and D in (64, 128) and not qk_fp8:
+        flops = 2.0 * B * H * rt * N * (D + Dv)
+        if num_iters > 1 and D == Dv and (D == 128 or D == 64 and flops < _PAIR_64_MAX_FLOPS) and not qk_fp8:
             order = "with_r0"
         else:
-            order = "start" if 2.0 * B * H * rt * N * (D + Dv) >= _FORK_MIN_FLOPS else "off"
+            order = "start" if flops >= _FORK_MIN_FLOPS else "off"
     return _OVERLAPS[order], _recompute_splits(B * H, rt, N, order == "with_r0")
 
 
@@ -163,14 +164,21 @@ def _fused_supported(q, k, v, num_blocks):
 # Where the exact recompute of the first rt queries runs: it reads q, k, v only and writes rows [0, rt) of z, which
 # the L-steps never write, so it can run beside the R/L chain.  "with_r0": its workgroups in one launch with R-step
 # 0's; "start" / "after_r0" / "after_r1": on a second stream, forked there and joined at the end; "off": after the
-# chain; "auto": with_r0 where that launch is built (more than one iteration, equal head dims of 64 or 128, no fp8 S),
-# otherwise start from _FORK_MIN_FLOPS on, else off.  Fork and join cost ~45 us of host time in the HIP runtime
-# (event records and cross-stream waits), which small calls waited for; the shared launch costs none.  Whole
+# chain; "auto": with_r0 where that launch is built (more than one iteration, equal head dims of 64 or 128, no fp8 S)
+# and 64-wide exact rows take less than _PAIR_64_MAX_FLOPS; otherwise start from _FORK_MIN_FLOPS on, else off.  Fork
+# and join cost ~45 us of host time in the HIP runtime (event records and cross-stream waits), which small calls
+# waited for; the shared launch costs none.  Whole
 # forward, us, start / off / with_r0: 4 x 64 grid, 2 heads 59.8 / 25.7 / 21.2; 16 x 256, 8 problems 66.8 / 67.4 / 57.7;
 # 21 x 400, 12 heads 150.6 / 157.1 / 151.4; 21 x 800 386.8 / 389.9 / 380.3; 33 x 993 902 / 909 / 889; 21 x 1560
-# 1181 / 1194 / 1176.
+# 1181 / 1194 / 1176.  At 64-wide heads R-step 0 alone has three workgroups per CU (146 registers) and in the shared
+# launch two (the exact rows' 171), so there the fork wins once its host time is hidden, start / with_r0: 12 heads,
+# 4 x 1200 (17.7 GFLOP of exact rows) 110 / 121, 4 x 1560 164 / 172, 33 x 700 292 / 300, 48 x 682 394 / 407, 21 x 1560
+# 637 / 648, 24 heads 1265 / 1303; level at 17.2 (2 x 2048, 8 heads) 110.6 / 111.6, 33 x 400 149 / 149, 21 x 800 215 /
+# 213, 21 x 1100 357 / 355; 4.0 (8 x 700, 4 heads) 64 / 55.  128-wide (two workgroups per CU either way): shared 0-9%
+# faster but for 4 x 1200 (183 / 188).
 _RECOMPUTE_OVERLAP = "auto"
 _FORK_MIN_FLOPS = 4e9   # (~the same figures: 16 x 256, 4.3 GFLOP of exact rows, start and off are level)
+_PAIR_64_MAX_FLOPS = 16e9
 _OVERLAPS = {"off": 0, "start": 1, "after_r0": 2, "after_r1": 3, "with_r0": 4}
 _side_streams = {}
 
