@@ -63,7 +63,7 @@ constexpr float kFp8Max = 448.f;   // e4m3's largest finite value (the conversio
 // per CU (64 / 128: spills, so one; now 229 registers) or spills (128 / 64: 13, now none).  64 / 128, fp16, us at three
 // slots and one workgroup per CU -> two and two: 48 heads x 777 tokens 34.3 -> 24.8, 24 x 8192 793 -> 647; 32 / 64, bf16,
 // 12 x 4096 110 -> 77; 128 / 64, 48 x 777 26.1 -> 24.3.
-constexpr int fwd_slots(int stage_bytes, int waves) {
+constexpr int fwd_slots(int stage_bytes) {
   return 3 * stage_bytes <= 64 * 1024 ? 3 : 2;
 }
 

@@ -53,7 +53,7 @@ __device__ __forceinline__ void fea_fwd_tile(const FwdParams& p, const int L) {
   constexpr int W1_BYTES = kFwdBN * DW1K * 2;
   constexpr int K8_OFF = K_BYTES + W0_BYTES + W1_BYTES;   // the fp8 K tile (QK8)
   constexpr int STAGE = fwd_stage_bytes<D, DW0, DW1, W0K, QK8>();
-  constexpr int NSLOT = fwd_slots(STAGE, WAVES);
+  constexpr int NSLOT = fwd_slots(STAGE);
   static_assert(!QK8 || D == 128, "fp8 S is built for 128-wide q / k");
   constexpr int kBM = 32 * kFwdQB * WAVES;   // queries per workgroup
   constexpr int NA0 = DW0K / 32;
@@ -642,13 +642,9 @@ __device__ __forceinline__ void fea_fwd_tile(const FwdParams& p, const int L) {
   }
 }
 
-// XCD-aware block -> tile map: block b runs on XCD b % 8, so give each XCD a contiguous run of
-// logical tiles (all query tiles of a problem then share one L2 for their K / W traffic).
-__device__ __forceinline__ int fwd_logical(int block, int grid) { return (block & 7) * (grid >> 3) + (block >> 3); }
-
 template <bool F16, int D, int DW0, int DW1, bool W0K, int ENT, bool SPLIT, int WAVES, bool QK8>
 __global__ __launch_bounds__(64 * WAVES, (fwd_min_blocks<D, DW0, DW1, ENT, WAVES>())) void fea_fwd_kernel(FwdParams p) {
-  const int L = fwd_logical(blockIdx.x, gridDim.x);
+  const int L = xcd_remap(blockIdx.x, gridDim.x);   // (all query tiles of a problem share one L2 for their K / W traffic)
   if (L < p.total_wg) fea_fwd_tile<F16, D, DW0, DW1, W0K, ENT, SPLIT, WAVES, QK8>(p, L);
 }
 
@@ -658,10 +654,10 @@ template <bool F16, int D, bool SPLIT>
 __global__ __launch_bounds__(64 * kFwdWavesSmall, 2) void fea_fwd_pair_kernel(FwdParams a, FwdParams b, int grid_a) {
   const int blk = blockIdx.x;
   if (blk < grid_a) {
-    const int L = fwd_logical(blk, grid_a);
+    const int L = xcd_remap(blk, grid_a);
     if (L < a.total_wg) fea_fwd_tile<F16, D, D, 0, false, kEntNone, SPLIT, kFwdWavesSmall, false>(a, L);
   } else {
-    const int L = fwd_logical(blk - grid_a, (int)gridDim.x - grid_a);
+    const int L = xcd_remap(blk - grid_a, (int)gridDim.x - grid_a);
     if (L < b.total_wg) fea_fwd_tile<F16, D, D, 0, true, kEntFromPK, false, kFwdWavesSmall, false>(b, L);
   }
 }
@@ -746,8 +742,7 @@ __global__ __launch_bounds__(256) void fea_fp8_keys_kernel(FwdParams p) {
 template <bool F16, int D, int DW0, int DW1, bool W0K, int ENT, bool SPLIT, int WAVES, bool QK8 = false>
 static int launch_fwd(FwdParams p, hipStream_t stream) {
   constexpr int STAGE = fwd_stage_bytes<D, DW0, DW1, W0K, QK8>();
-  constexpr int LDS = fwd_slots(STAGE, WAVES) * STAGE > WAVES * kEpiPatchBytes ? fwd_slots(STAGE, WAVES) * STAGE
-                                                                              : WAVES * kEpiPatchBytes;
+  constexpr int RING = fwd_slots(STAGE) * STAGE, LDS = RING > WAVES * kEpiPatchBytes ? RING : WAVES * kEpiPatchBytes;
   constexpr int BM = 32 * kFwdQB * WAVES;
   p.q_tiles = (p.nq + BM - 1) / BM;
   p.total_wg = p.problems * p.splits * p.q_tiles;
@@ -778,7 +773,7 @@ static int launch_fwd(FwdParams p, hipStream_t stream) {
 template <bool F16, int D, bool SPLIT>
 static int launch_pair(FwdParams a, FwdParams b, hipStream_t stream) {
   constexpr int SA = fwd_stage_bytes<D, D, 0, false, false>(), SB = fwd_stage_bytes<D, D, 0, true, false>();
-  constexpr int LA = fwd_slots(SA, kFwdWavesSmall) * SA, LB = fwd_slots(SB, kFwdWavesSmall) * SB, LDS = LA > LB ? LA : LB;
+  constexpr int LA = fwd_slots(SA) * SA, LB = fwd_slots(SB) * SB, LDS = LA > LB ? LA : LB;
   static_assert(LDS <= 65536 && LDS >= kFwdWavesSmall * kEpiPatchBytes, "LDS within the default limit");
   constexpr int BM = 32 * kFwdQB * kFwdWavesSmall;
   for (FwdParams* p : {&a, &b}) {

@@ -82,12 +82,11 @@ __device__ __forceinline__ int swz_rows(int r) {
   else return ((r & 3) << 2) | ((r >> 2) & 3);
 }
 
-// XCD-aware block order for a grid of nblocks (a multiple of 8): block b runs on XCD b % 8, so give
-// each XCD a contiguous run of logical blocks (neighbouring tiles / rows then share that XCD's L2).
-__device__ __forceinline__ int xcd_remap(int nblocks) {
-  const int per_xcd = nblocks >> 3;
-  return (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-}
+// XCD-aware block order for a grid (or a part of one that starts at a multiple of 8) of nblocks, a multiple of 8: block
+// b runs on XCD b % 8, so give each XCD a contiguous run of logical blocks (neighbouring tiles / rows then share that
+// XCD's L2).
+__device__ __forceinline__ int xcd_remap(int block, int nblocks) { return (block & 7) * (nblocks >> 3) + (block >> 3); }
+__device__ __forceinline__ int xcd_remap(int nblocks) { return xcd_remap((int)blockIdx.x, nblocks); }
 
 __device__ __forceinline__ float wave_max32(float x) {
   // combine lane l with lane l ^ 32
