@@ -1,7 +1,7 @@
 // FlashEntropyAttention forward for launches with few query tiles (gfx950).
 //
-// The 128-query kernel (fea_fwd.hip) walks a problem's keys serially in 64-key stages of ~0.45 us (64-wide heads) to
-// 0.55 us (128-wide), so a launch of few tiles takes one workgroup's whole key loop while most CUs idle: (1, 2,
+// The 128-query kernel (fea_fwd.hip) walks a problem's keys serially in 64-key stages of ~0.8 us (64-wide heads) to
+// ~1.05 us (128-wide) with one workgroup to the CU, so a launch of few tiles takes one workgroup's whole key loop while most CUs idle: (1, 2,
 // 1024, 64) was 16 workgroups of 16 stages, 16.8 us.  Here a workgroup takes fewer queries and its waves split the
 // keys: wave (qg, kg) of QG x KG takes query block qg (32 queries) and the 32-key block kg of every stage of 32 KG
 // keys, with its own sums and accumulators, all relative to the row's one reference point; a tree over the key

@@ -2,15 +2,17 @@
 // results and workspaces from torch's caching allocator and issues the launch sequences of the flash-entropy and
 // VMonarch attention, forward and backward.
 //
-// Why native: a VMonarch forward is six launches plus the fork and join of the recompute's stream.  Issued from
-// Python through ctypes each launch cost ~20 us of host time (struct fields, views, allocations, stream queries)
-// against 4-20 us of GPU time at small sizes, so small calls ran at the host's pace: back to back on one box, a
-// VMonarch forward of a 4 x 64 grid took 135 us and takes 61, of a 16 x 256 grid (batch 2, 4 heads) 139 and 70, a
-// flash-entropy forward (1, 2, 1024, 64) 30 and 17, its training step at (2, 4, 1000, 64) 224 and 115.
+// Why native: a VMonarch forward of two iterations is five or six launches (R- and L-steps, the exact recompute beside
+// R-step 0, the merge of its key ranges where it has several), in some orders with a second stream's fork and join.
+// Issued from Python through ctypes each launch cost ~20 us of host time (struct fields, views, allocations, stream
+// queries) against 4-20 us of GPU time at small sizes, so small calls ran at the host's pace.  Back to back on one box,
+// the same launches from Python -> from here, in us: VMonarch forward of a 4 x 64 grid 135 -> 61, of 16 x 256 (batch 2,
+// 4 heads) 139 -> 70 (with the recompute in R-step 0's launch, without the fork: 21 and 58); flash-entropy forward
+// (1, 2, 1024, 64) 30 -> 17 (key-group kernel: 9.6), its training step at (2, 4, 1000, 64) 224 -> 115.
 //
 // Every call only issues work on the current stream (and the given side stream, joined before returning); nothing
-// is kept between calls, and no check is cached.  The C ABI it calls (include/vmonarch_amd.h) validates its
-// arguments before launching.
+// is kept between calls, and no check is cached.  Types and devices are checked here, sizes, strides and alignment by
+// the C ABI (include/vmonarch_amd.h), all before a launch.
 #include <Python.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
