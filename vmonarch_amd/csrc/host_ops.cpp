@@ -70,9 +70,9 @@ c10::DeviceGuard on_gpu_of(const Tensor& q) {
   if (!q.is_cuda()) throw py::value_error("vmonarch_amd: needs GPU tensors, got " + q.device().str());
   return c10::DeviceGuard(q.device());
 }
-void same_device(const Tensor& q, const Tensor& t) { require(t.device() == q.device(), "all tensors on q's device"); }
+void same_device(const Tensor& q, const Tensor& t) { require(t.device() == q.device(), "all tensors on one GPU: q's device"); }
 void like(const Tensor& q, const Tensor& t) {
-  require(t.scalar_type() == q.scalar_type(), "all of q's dtype");
+  require(t.scalar_type() == q.scalar_type(), "all of one dtype: q's");
   same_device(q, t);
 }
 void like(const Tensor& q, std::initializer_list<const Tensor*> ts) {

@@ -107,14 +107,14 @@ def _recorded(*tensors):
 
 def _plain_call(q, k, v):
     """Whether flash_entropy_attention can go straight to the kernels: nothing records the call (autograd's function,
-    ~12 us of host time, is then only passed through), and inputs that its forward takes as they are."""
+    ~12 us of host time, is then only passed through), and inputs that its forward takes as they are (the host module
+    asks for one dtype and device itself)."""
     if _recorded(q, k, v):
         return False
     if not (type(q) is type(k) is type(v) is torch.Tensor and q.is_cuda and q.dim() == 4):
         return False
     D, Dv = q.shape[-1], v.shape[-1]
-    return (q.dtype in _lib.DTYPES and k.dtype == v.dtype == q.dtype and k.device == v.device == q.device
-            and k.shape == q.shape and v.shape[:-1] == q.shape[:-1] and D in _HEAD_DIMS
+    return (q.dtype in _lib.DTYPES and k.shape == q.shape and v.shape[:-1] == q.shape[:-1] and D in _HEAD_DIMS
             and Dv in _HEAD_DIMS and not (D == 256 and Dv != 256) and _kernel_widths(D, Dv) == (D, Dv))
 
 
