@@ -15,6 +15,7 @@
 // the C ABI (include/vmonarch_amd.h), all before a launch.
 #include <Python.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
@@ -65,11 +66,14 @@ int dtype_code(const Tensor& t) {
 
 // The kernels take every tensor's type and place from q, so a tensor of another type would be read as what it is not, and
 // one elsewhere through an address the GPU does not have.
-// on_gpu_of(q): q's GPU is the current one while the result lives, as a null stream and an event's creation take that.
-c10::DeviceGuard on_gpu_of(const Tensor& q) {
-  if (!q.is_cuda()) throw py::value_error("vmonarch_amd: needs GPU tensors, got " + q.device().str());
-  return c10::DeviceGuard(q.device());
-}
+// OnGpuOf(q): q's GPU is the current one while this lives, as a null stream and an event's creation take that.
+struct OnGpuOf {
+  c10::OptionalDeviceGuard guard;
+  explicit OnGpuOf(const Tensor& q) {
+    if (!q.is_cuda()) throw py::value_error("vmonarch_amd: needs GPU tensors, got " + q.device().str());
+    if (c10::hip::current_device() != q.device().index()) guard.reset_device(q.device());
+  }
+};
 void same_device(const Tensor& q, const Tensor& t) { require(t.device() == q.device(), "all tensors on one GPU: q's device"); }
 void like(const Tensor& q, const Tensor& t) {
   require(t.scalar_type() == q.scalar_type(), "all of one dtype: q's");
@@ -200,7 +204,6 @@ const Tensor* ptr(const OptT& t) { return t ? &*t : nullptr; }
 std::tuple<Tensor, OptT, OptT> fea_fwd(const Tensor& q, const Tensor& k, const Tensor& w0, const OptT& w1, double sm_scale,
                                        int64_t frames, OptT o, OptT lse, OptT ent, bool want_ent, bool want_lse,
                                        int64_t num_splits, bool qk_fp8) {
-  const c10::DeviceGuard device = on_gpu_of(q);
   const int64_t B = q.size(0), H = q.size(1), NQ = q.size(2);
   if (!o) o = at::empty({B, H, NQ, w0.size(3) + (w1 ? w1->size(3) : 0)}, q.options());
   if (!lse && want_lse) lse = at::empty({B, H, NQ}, f32(q));
@@ -263,7 +266,6 @@ std::tuple<Tensor, Tensor, OptT> fea_bwd(const Tensor& q, const Tensor& k, const
                                          OptT dk, OptT dv, const std::string& overwrite, const OptT& v1, bool fold_k,
                                          const OptT& dk_base, const OptT& dv_base, int64_t frames, int64_t route_flags,
                                          const OptT& dq_base, const OptT& delta) {
-  const c10::DeviceGuard device = on_gpu_of(q);
   int32_t flags = (fold_k ? VMO_BWD_FOLD_K : 0) | (int32_t)route_flags;
   struct G { const OptT& t; char name; int accum, f32_bit, sum; const OptT& base; };
   for (const G& g : {G{dq, 'q', VMO_BWD_ACCUM_Q, VMO_BWD_F32_Q, VMO_BWD_SUM_Q, dq_base},
@@ -290,7 +292,6 @@ std::tuple<Tensor, Tensor, OptT> fea_bwd(const Tensor& q, const Tensor& k, const
 
 void lstep_fwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tensor& res, int64_t m, int64_t b, double scale,
                bool last, int64_t skip, double min_col_mass) {
-  const c10::DeviceGuard device = on_gpu_of(q);
   like(q, {&out, &res});
   same_device(q, ent);
   vmo_lstep_args a{};
@@ -308,7 +309,6 @@ void lstep_fwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tens
 void lstep_bwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tensor& grad_res, const Tensor& grad_q,
                const Tensor& grad_out, int64_t m, int64_t b, double scale, bool last, int64_t skip, double min_col_mass,
                bool overwrite_q, const OptT& delta) {
-  const c10::DeviceGuard device = on_gpu_of(q);
   like(q, {&out, &grad_res, &grad_out});
   require(grad_q.scalar_type() == at::kFloat, "grad_q: float32");
   same_device(q, {&ent, &grad_q, ptr(delta)});
@@ -334,7 +334,7 @@ void lstep_bwd(const Tensor& q, const Tensor& out, const Tensor& ent, const Tens
 
 std::tuple<Tensor, Tensor, Tensor> fea_attention(const Tensor& q0, const Tensor& k0, const Tensor& v0, double sm_scale) {
   like(q0, {&k0, &v0});
-  const c10::DeviceGuard device = on_gpu_of(q0);
+  const OnGpuOf device(q0);
   const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0);
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2);
   Tensor o = empty_in_layout(q0, v.size(3));
@@ -347,7 +347,7 @@ std::tuple<Tensor, Tensor, Tensor> fea_attention_bwd(const Tensor& q0, const Ten
                                                      const Tensor& lse, const Tensor& ent, const Tensor& do0,
                                                      const Tensor& dE, double sm_scale) {
   like(q0, {&k0, &v0, &o0, &do0});
-  const c10::DeviceGuard device = on_gpu_of(q0);
+  const OnGpuOf device(q0);
   // the gradients in the memory order of the caller's q, k, v
   Tensor dq = empty_in_layout(q0, q0.size(3)), dk = empty_in_layout(k0, k0.size(3)), dv = empty_in_layout(v0, v0.size(3));
   const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0), o = row_aligned(o0), dO = row_aligned(do0);
@@ -403,7 +403,7 @@ Tensor vmonarch_fwd(const Tensor& q0, const Tensor& k0, const Tensor& v0, int64_
                     int64_t recompute_tokens, double min_col_mass, double scale, bool qk_fp8, int64_t splits, int overlap,
                     int64_t side_handle, const Stages& stage) {
   like(q0, {&k0, &v0});
-  const c10::DeviceGuard device = on_gpu_of(q0);
+  const OnGpuOf device(q0);
   const Tensor q = row_aligned(q0), k = row_aligned(k0), v = row_aligned(v0);
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Dv = v.size(3);
   const int64_t rt = std::min<int64_t>(recompute_tokens, N);
@@ -464,7 +464,7 @@ std::tuple<std::vector<int>, std::vector<Tensor>> vmonarch_fwd_train(const Tenso
                                                                      double min_col_mass, double scale, int64_t splits,
                                                                      int overlap, int64_t side_handle) {
   like(q0, {&k0, &v0});
-  const c10::DeviceGuard device = on_gpu_of(q0);
+  const OnGpuOf device(q0);
   std::vector<int> orders;
   for (const Tensor* t : {&q0, &k0, &v0})
     for (int d : layout_order(*t)) orders.push_back(d);
@@ -525,7 +525,7 @@ std::tuple<Tensor, Tensor, Tensor> vmonarch_bwd(const std::vector<int>& orders, 
                                                 int64_t m, int64_t b, int64_t iters, int64_t rt, double min_col_mass,
                                                 double scale, int want_delta) {
   const Tensor &q = all[0], &k = all[1], &v = all[2], &z = all[3], &lse_rt = all[4];
-  const c10::DeviceGuard device = on_gpu_of(q);
+  const OnGpuOf device(q);
   same_device(q, dz0);
   const Tensor dz = row_aligned(dz0.to(q.scalar_type()));
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3), Dv = v.size(3);
@@ -583,14 +583,23 @@ std::tuple<Tensor, Tensor, Tensor> vmonarch_bwd(const std::vector<int>& orders, 
   return {gq, gk, gv};
 }
 
+// A single launch as an entry of its own: on its first tensor's GPU.
+template <class R, class... A>
+auto on_its_gpu(R (*launch)(const Tensor&, A...)) {
+  return [launch](const Tensor& q, A... rest) -> R {
+    const OnGpuOf device(q);
+    return launch(q, std::forward<A>(rest)...);
+  };
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, mod) {
   using NoGil = py::call_guard<py::gil_scoped_release>;
-  mod.def("fea_fwd", &fea_fwd, NoGil());
-  mod.def("fea_bwd", &fea_bwd, NoGil());
-  mod.def("lstep_fwd", &lstep_fwd, NoGil());
-  mod.def("lstep_bwd", &lstep_bwd, NoGil());
+  mod.def("fea_fwd", on_its_gpu(&fea_fwd), NoGil());
+  mod.def("fea_bwd", on_its_gpu(&fea_bwd), NoGil());
+  mod.def("lstep_fwd", on_its_gpu(&lstep_fwd), NoGil());
+  mod.def("lstep_bwd", on_its_gpu(&lstep_bwd), NoGil());
   mod.def("fea_attention", &fea_attention, NoGil());
   mod.def("fea_attention_bwd", &fea_attention_bwd, NoGil());
   mod.def("vmonarch_fwd", [](const Tensor& q, const Tensor& k, const Tensor& v, int64_t m, int64_t b, int64_t iters,
